@@ -43,6 +43,10 @@ ChainDims chain_dims(int rows, int cols, int orient_tall);
 int chain_check(const char* what, const ChainDims& d);
 ChainWs chain_ws(void* ws, int batch, const ChainDims& d);   // ws == nullptr: sizes only
 
+// The rows and columns of T0 (from the first; multiples of 64) that an entry has to write
+// for chain_run_packed on this batch, its zero padding included.
+void chain_extent(const ChainDims& d, int batch, int* rows, int* cols);
+
 // Run `steps` iterations from T0 already packed in the workspace; the result
 // goes to `out` (batch, rows, cols) bf16 in the orientation given.
 int chain_run_packed(hipStream_t stream, const ChainWs& w, int batch, const ChainDims& d,

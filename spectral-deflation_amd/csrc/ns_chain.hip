@@ -125,6 +125,8 @@ struct GemmArgs {
   int total_tiles;                               // over the batch
   int batch, rev;                                // rev: walk the batch from its last matrix
   int kspread;                                   // K walk starts at stage kspread (ti + tj) mod nk
+  int kvalid, ref_tile;                          // gemm_tile64: K without its zero padding, and the
+                                                 // tile size whose K walk it follows
   float alpha, beta;                             // POLY: (b, c)
   float diag_add; int diag_lim;                  // POLY: + diag_add on C[i][i], i < diag_lim
   const bf16* aux; long long aux_bs; int aux_rows; // POLY: A (indexed [i][j])
@@ -700,6 +702,319 @@ void gemm_nt_bf16(GemmArgs g) {
 #undef DMH_SCHED_SUB
 #undef DMH_GLOAD
 }
+
+// ---------------------------------------------------------------------------
+// The same products for matrices too few or too small to give the compute units several
+// 256 x 256 (or 128 x 128) tiles each: smaller output tiles, one per workgroup, with a
+// deeper ring.  A lone workgroup is bound by the latency of its stage loads (a 2-slot
+// ring has one stage in flight), so NS stages are, and by LDS reads, which a wave of one
+// 32 x 32 block needs 2 KB of per MFMA.  Chain of five iterations with its entry, against
+// gemm_nt_bf16 (one box): one (192, 96) 146 -> 65 us, (1000, 333) 228 -> 93, (3072, 768)
+// 412 -> 178, 3 x (1280, 1280) 527 -> 310, (5120, 1280) 897 -> 330; at (3072, 768) K1 takes
+// 14.9 us (78 tiles of 48 stages, 12 us with one tile alone: ~0.2 us a stage for the
+// barrier, the fragment reads and the MFMAs), K2 7.8, K3 11.  At (192, 96) each launch is
+// ~3.7 us, its floor.
+//
+// Every output sums the same products in the same order as gemm_nt_bf16 (the same MFMA
+// over the same K walk, started where the tile of `ref_tile` that holds this one starts
+// it; K stages that are all padding add zeros and are left out), so the kernels agree
+// bit for bit and the choice between them may depend on the batch.
+// ---------------------------------------------------------------------------
+template <int WM_, int WN_, int BM_, int BN_, int NS_>
+struct RingCfg {
+  static constexpr int WM = WM_, WN = WN_, BM = BM_, BN = BN_, NS = NS_;
+  static constexpr int NW = WM * WN, THREADS = 64 * NW;
+  static constexpr int TM = 32 * BM * WM, TN = 32 * BN * WN;   // output tile
+  static constexpr int PB = TM * ROWB, QB = TN * ROWB;         // bytes per operand and stage
+  static constexpr int STAGEB = PB + QB;
+  static constexpr int LP = PB / (1024 * NW), LQ = QB / (1024 * NW);   // loads per wave and stage
+  static constexpr int LPS = LP + LQ;
+  static constexpr int PITCH = TN + 4;                         // epilogue rows (bf16)
+  static constexpr int CH = TM * TN / 8 / THREADS;             // 16-byte output chunks per thread
+  static_assert(LP * 1024 * NW == PB && LQ * 1024 * NW == QB, "whole loads per wave");
+  static_assert(LPS * (NS - 1) < 64, "vmcnt counts the loads in flight");
+  static_assert(TM * PITCH * 2 <= NS * STAGEB, "the epilogue reuses the ring");
+  static_assert(NS * STAGEB <= 160 * 1024, "the ring must fit the LDS");
+};
+
+// s_waitcnt vmcnt(n), expcnt and lgkmcnt left at their maxima
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
+// ... for n = k * STEP, k < NS
+template <int STEP, int NS>
+__device__ __forceinline__ void wait_stages(int k) {
+  static_assert(NS <= 8, "cases");
+  switch (k) {
+    case 7: if constexpr (NS > 7) { wait_vmcnt<7 * STEP>(); break; }
+    case 6: if constexpr (NS > 6) { wait_vmcnt<6 * STEP>(); break; }
+    case 5: if constexpr (NS > 5) { wait_vmcnt<5 * STEP>(); break; }
+    case 4: if constexpr (NS > 4) { wait_vmcnt<4 * STEP>(); break; }
+    case 3: if constexpr (NS > 3) { wait_vmcnt<3 * STEP>(); break; }
+    case 2: if constexpr (NS > 2) { wait_vmcnt<2 * STEP>(); break; }
+    case 1: wait_vmcnt<STEP>(); break;
+    default: wait_vmcnt<0>(); break;
+  }
+}
+
+// grid: batch * tiles, one tile each
+template <int EPI, int TNL, class C>
+__global__ __launch_bounds__(C::THREADS) void gemm_ring(GemmArgs g) {
+  constexpr int WN = C::WN, BM = C::BM, BN = C::BN, NS = C::NS, TM = C::TM, TN = C::TN;
+  constexpr int LP = C::LP, LQ = C::LQ, CH = C::CH, PITCH = C::PITCH;
+  __shared__ __attribute__((aligned(1024))) char smem[NS * C::STAGEB];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lid = xcd_remap(blockIdx.x, gridDim.x);
+  int b, ti, tj;
+  if (g.sym) {   // (square tiles) upper triangle by rows: row ti starts at ti T - ti (ti - 1) / 2
+    const int T = g.tiles_m, per = T * (T + 1) / 2;
+    b = lid / per;
+    const int rem = lid - b * per;
+    const float h = T + 0.5f;
+    ti = (int)(h - sqrtf(fmaxf(h * h - 2.f * rem, 0.f)));
+    ti = ti < 0 ? 0 : (ti > T - 1 ? T - 1 : ti);
+    while (ti > 0 && ti * T - ti * (ti - 1) / 2 > rem) --ti;
+    while (ti + 1 < T && (ti + 1) * T - (ti + 1) * ti / 2 <= rem) ++ti;
+    tj = ti + rem - (ti * T - ti * (ti - 1) / 2);
+  } else {
+    const int per = g.tiles_m * g.tiles_n;
+    b = lid / per;
+    const int t = lid - b * per;
+    ti = t / g.tiles_n;
+    tj = t - ti * g.tiles_n;
+  }
+  const int i0 = ti * TM, j0 = tj * TN;
+
+  // POLY: this thread's chunks of the aux tile, requested first
+  bf16x8 av[EPI == EPI_POLY ? CH : 1];
+  if (EPI == EPI_POLY) {
+    const bf16* ab = g.aux + (long long)b * g.aux_bs;
+#pragma unroll
+    for (int v = 0; v < CH; ++v) {
+      const int u = tid + C::THREADS * v, r = u / (TN / 8), ch = u % (TN / 8);
+      av[v] = *(const bf16x8*)(ab + blk_off(i0 + r, j0 + 8 * ch, g.aux_rows));
+    }
+  }
+
+  // A stage of an operand is W = TM or TN rows x 64 k (rows), or 64 k x W columns (K-major);
+  // stage ks is `step` bytes further.  LDS holds it as rows of 128 bytes (rows) or 2 W bytes
+  // (K-major), filled 1 KB per load in order; 16-byte chunk c of row r sits in slot c ^ swz(r).
+  // rows: lds_swz, as in gemm_nt_bf16.  K-major: half a transposing read takes 64 bytes of
+  // four consecutive rows, which the swizzle puts into distinct quarters of the 256 bytes
+  // that the banks hold.
+  const int nk = g.K / TK, nkv = (g.kvalid + TK - 1) / TK;
+  const int stepP = TNL ? CHAIN_BLK * ROWB : g.p_rows * ROWB;
+  const int stepQ = TNL ? CHAIN_BLK * ROWB : g.q_rows * ROWB;
+  const bf16* Pb = g.P + (long long)b * g.p_bs + (TNL ? blk_off(0, i0, g.p_rows) : blk_off(i0, 0, g.p_rows));
+  const bf16* Qb = g.Q + (long long)b * g.q_bs + (TNL ? blk_off(0, j0, g.q_rows) : blk_off(j0, 0, g.q_rows));
+  // (record counts: to the end of the last stage's last row)
+  const __amdgpu_buffer_rsrc_t rP = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)Pb, (short)0,
+      TNL ? ((TM - 1) / 64 * g.p_rows + g.p_rows) * ROWB - (i0 & 63) * 2
+          : (nk - 1) * stepP + TM * ROWB, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rQ = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)Qb, (short)0,
+      TNL ? ((TN - 1) / 64 * g.q_rows + g.q_rows) * ROWB - (j0 & 63) * 2
+          : (nk - 1) * stepQ + TN * ROWB, 0x00020000);
+  auto swz = [](int r, int W) {
+    if (!TNL) return lds_swz(r);
+    return W == 32 ? 0 : (W == 64 ? 4 * ((r >> 1) & 1) : 4 * (r & 3));
+  };
+  auto load_off = [&](int q, int W, int L, int rows) {   // of load q of this wave's L
+    const int u = (wave * L + q) * 64 + lane;
+    if (TNL) {
+      const int cpr = W / 8, r = u / cpr, c = (u % cpr) ^ swz(r, W);
+      return (c >> 3) * rows * ROWB + r * ROWB + (c & 7) * 16;
+    }
+    const int r = u / CHUNKS;
+    return r * ROWB + ((u % CHUNKS) ^ swz(r, W)) * 16;
+  };
+  int voffP[LP], voffQ[LQ];
+#pragma unroll
+  for (int q = 0; q < LP; ++q) voffP[q] = load_off(q, TM, LP, g.p_rows);
+#pragma unroll
+  for (int q = 0; q < LQ; ++q) voffQ[q] = load_off(q, TN, LQ, g.q_rows);
+  char* const ldsP = smem + wave * LP * 1024;
+  char* const ldsQ = smem + C::PB + wave * LQ * 1024;
+  const int wm = wave / WN, wn = wave % WN, r32 = lane & 31, hi = lane >> 5;
+  auto frag_off = [&](int c0, int st, int W) {
+    if (TNL) {
+      const int gq = lane >> 4, e = (lane >> 2) & 3, q = lane & 3;
+      const int k = 16 * st + 8 * (gq >> 1) + e;
+      const int c = c0 + 16 * (gq & 1) + 4 * q;
+      return k * 2 * W + (((c >> 3) ^ swz(k, W)) * 16) + (c & 7) * 2;
+    }
+    const int row = c0 + r32;
+    return row * ROWB + ((2 * st + hi) ^ swz(row, W)) * 16;
+  };
+  int offP[BM][KSUB], offQ[BN][KSUB];
+#pragma unroll
+  for (int st = 0; st < KSUB; ++st) {
+#pragma unroll
+    for (int i = 0; i < BM; ++i) offP[i][st] = frag_off(32 * (BM * wm + i), st, TM);
+#pragma unroll
+    for (int j = 0; j < BN; ++j) offQ[j][st] = C::PB + frag_off(32 * (BN * wn + j), st, TN);
+  }
+  bf16x8 fp[2][KSUB][BM], fq[2][KSUB][BN];
+  auto read = [&](int slot, int x) {
+    const char* base = smem + slot * C::STAGEB;
+#pragma unroll
+    for (int st = 0; st < KSUB; ++st) {
+#pragma unroll
+      for (int i = 0; i < BM; ++i)
+        fp[x][st][i] = TNL ? lds_tr_frag(base + offP[i][st], 2 * TM)
+                           : *(const bf16x8*)(base + offP[i][st]);
+#pragma unroll
+      for (int j = 0; j < BN; ++j)
+        fq[x][st][j] = TNL ? lds_tr_frag(base + offQ[j][st], 2 * TN)
+                           : *(const bf16x8*)(base + offQ[j][st]);
+    }
+  };
+
+  // K walk: stages k0, k0 + 1, ..., nkv - 1, 0, ..., k0 - 1
+  int k0 = (g.kspread * (i0 / g.ref_tile + j0 / g.ref_tile)) % nk;
+  if (k0 >= nkv) k0 = 0;
+  int issued = 0, ks_next = k0, slot_next = 0;
+  auto issue_next = [&]() {
+    const int so = slot_next * C::STAGEB;
+#pragma unroll
+    for (int q = 0; q < LP; ++q) load_lds16(rP, ldsP + so + q * 1024, voffP[q], ks_next * stepP);
+#pragma unroll
+    for (int q = 0; q < LQ; ++q) load_lds16(rQ, ldsQ + so + q * 1024, voffQ[q], ks_next * stepQ);
+    ++issued;
+    ks_next = ks_next + 1 == nkv ? 0 : ks_next + 1;
+    slot_next = slot_next + 1 == NS ? 0 : slot_next + 1;
+  };
+  // every wave's loads of a stage have landed, and its reads of the one before are done
+  // (the builtin wait, which the compiler's own tracking sees: it then adds none before the
+  // MFMAs for the fragments read in the step before)
+  auto barrier = [&]() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
+    if (C::NW > 1) __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  f32x16 acc[BM][BN];
+#pragma unroll
+  for (int i = 0; i < BM; ++i)
+#pragma unroll
+    for (int j = 0; j < BN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  for (int s = 0; s < NS && s < nkv; ++s) issue_next();
+  wait_stages<C::LPS, NS>(issued - 1);
+  barrier();
+  read(0, 0);
+  int slot = 0;   // of stage s
+  auto mma = [&](int x) {
+#pragma unroll
+    for (int st = 0; st < KSUB; ++st)
+#pragma unroll
+      for (int i = 0; i < BM; ++i)
+#pragma unroll
+        for (int j = 0; j < BN; ++j)
+          acc[i][j] = mfma_32x32x16(fq[x][st][j], fp[x][st][i], acc[i][j]);
+  };
+  // step s: once stage s + 1 has landed, its fragments are read under stage s's MFMAs, and
+  // stage s's slot (its fragments are in registers) takes stage s + NS.  The steps that still
+  // load run without branches, in pairs, so that the compiler keeps their reads in flight.
+  auto full_step = [&](int x) {
+    slot = slot + 1 == NS ? 0 : slot + 1;
+    wait_vmcnt<C::LPS * (NS - 2)>();
+    barrier();
+    read(slot, x ^ 1);
+    issue_next();
+    mma(x);
+  };
+  int s = 0;
+  for (; s + 1 + NS < nkv; s += 2) {
+    full_step(0);
+    full_step(1);
+  }
+  auto last_step = [&](int s, int x) {
+    if (s + 1 < nkv) {
+      slot = slot + 1 == NS ? 0 : slot + 1;
+      wait_stages<C::LPS, NS>(issued - (s + 2));
+      barrier();
+      read(slot, x ^ 1);
+      if (issued < nkv) issue_next();
+    }
+    mma(x);
+  };
+  for (; s + 1 < nkv; s += 2) {
+    last_step(s, 0);
+    last_step(s + 1, 1);
+  }
+  if (s < nkv) last_step(s, 0);
+
+  // epilogue: acc[i][j][4 g + q] holds C[32 i + r32][32 j + 8 g + 4 hi + q] of the wave's tile
+  __syncthreads();   // the ring is read out by every wave
+  bf16* const S = (bf16*)smem;
+#pragma unroll
+  for (int i = 0; i < BM; ++i)
+#pragma unroll
+    for (int j = 0; j < BN; ++j)
+#pragma unroll
+      for (int gq = 0; gq < 4; ++gq) {
+        bf16x4 o;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float v = acc[i][j][4 * gq + q];
+          o[q] = f2bf(EPI == EPI_POLY ? g.beta * v : v);
+        }
+        *(bf16x4*)(S + (32 * (BM * wm + i) + r32) * PITCH + 32 * (BN * wn + j) + 8 * gq + 4 * hi) = o;
+      }
+  __syncthreads();
+  const bool mirror = g.outT && !(g.sym && ti == tj);
+  if (g.out || EPI == EPI_POLY) {
+    bf16* outb = g.out + (long long)b * g.out_bs;
+    const bool al = g.out_rows > 0 || ((g.out_ld & 7) == 0 && (g.out_bs & 7) == 0 &&
+                                       (((uintptr_t)g.out) & 15) == 0);
+#pragma unroll
+    for (int v = 0; v < CH; ++v) {
+      const int u = tid + C::THREADS * v, r = u / (TN / 8), ch = u % (TN / 8);
+      const int gi = i0 + r, gj = j0 + 8 * ch;
+      bf16* sp = S + r * PITCH + 8 * ch;
+      const bf16x4 lo = *(const bf16x4*)sp, hi4 = *(const bf16x4*)(sp + 4);
+      bf16x8 val = __builtin_shufflevector(lo, hi4, 0, 1, 2, 3, 4, 5, 6, 7);
+      if (EPI == EPI_POLY) {
+        const int qd = ti == tj && gi < g.diag_lim ? gi - gj : -1;
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+          val[q] = f2bf(g.alpha * bf2f(av[EPI == EPI_POLY ? v : 0][q]) + bf2f(val[q]) +
+                        (q == qd ? g.diag_add : 0.f));
+        *(bf16x4*)sp = __builtin_shufflevector(val, val, 0, 1, 2, 3);
+        *(bf16x4*)(sp + 4) = __builtin_shufflevector(val, val, 4, 5, 6, 7);
+      }
+      if (gi >= g.valid_i || gj >= g.valid_j) continue;
+      const unsigned mask = gj + 8 > g.valid_j ? (1u << (g.valid_j - gj)) - 1u : 0xffu;
+      const long long off =
+          g.out_rows > 0 ? blk_off(gi, gj, g.out_rows) : (long long)gi * g.out_ld + gj;
+      store8(outb + off, val, mask, al);
+    }
+  }
+  if (!mirror) return;
+  if (EPI == EPI_POLY) __syncthreads();   // the polynomial's values replaced the staged ones
+  bf16* outtb = g.outT + (long long)b * g.outT_bs;
+  const bool alT = g.outT_rows > 0 || ((g.outT_ld & 7) == 0 && (g.outT_bs & 7) == 0 &&
+                                       (((uintptr_t)g.outT) & 15) == 0);
+#pragma unroll
+  for (int v = 0; v < CH; ++v) {
+    const int u = tid + C::THREADS * v, j = u / (TM / 8), ch = u % (TM / 8);
+    const int gj = j0 + j, gi = i0 + 8 * ch;
+    if (gj >= g.valid_j || gi >= g.valid_i) continue;
+    bf16x8 val;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) val[q] = S[(8 * ch + q) * PITCH + j];
+    const unsigned mask = gi + 8 > g.valid_i ? (1u << (g.valid_i - gi)) - 1u : 0xffu;
+    const long long off =
+        g.outT_rows > 0 ? blk_off(gj, gi, g.outT_rows) : (long long)gj * g.outT_ld + gi;
+    store8(outtb + off, val, mask, alT);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // entry: Frobenius norm partials, then scale + cast + pack into padded T and W
 // ---------------------------------------------------------------------------
@@ -955,6 +1270,46 @@ static int launch_gemm(const GemmArgs& g, int tile, int rows, int cols, int batc
                      : launch_gemm_tl<EPI, TNL, 256>(g, rows, cols, batch, stream, what);
 }
 
+// gemm_ring over rows x cols outputs per matrix (multiples of 64)
+template <int EPI, int TNL, class C>
+static int launch_ring_cfg(GemmArgs g, int rows, int cols, int batch, hipStream_t stream,
+                           const char* what) {
+  g.tiles_m = ceil_div(rows, C::TM);
+  g.tiles_n = ceil_div(cols, C::TN);
+  const long long per = g.sym ? (long long)g.tiles_m * (g.tiles_m + 1) / 2
+                              : (long long)g.tiles_m * g.tiles_n;
+  const long long tiles = per * batch;
+  if (tiles <= 0 || tiles > 0x7fffffffLL) {
+    set_error("%s: bad grid (%lld tiles)", what, tiles);
+    return DMH_EINVAL;
+  }
+  g.total_tiles = (int)tiles;
+  g.batch = batch;
+  hipLaunchKernelGGL((gemm_ring<EPI, TNL, C>), dim3((int)tiles), dim3(C::THREADS), 0, stream, g);
+  DMH_CHECK_LAUNCH(what);
+  return DMH_OK;
+}
+
+// gemm_ring configurations; tile (waves of blocks), ring depth, LDS
+enum { RING_NONE = 0, RING_64, RING_128x64, RING_128_DEEP, RING_128 };
+
+template <int EPI, int TNL>
+static int launch_ring(const GemmArgs& g, int cfg, int rows, int cols, int batch,
+                       hipStream_t stream, const char* what) {
+  switch (cfg) {
+    case RING_64:         // 2 x 2 waves of one 32 x 32 block, 4 slots, 64 KB
+      return launch_ring_cfg<EPI, TNL, RingCfg<2, 2, 1, 1, 4>>(g, rows, cols, batch, stream, what);
+    case RING_128x64:     // 2 x 2 waves of 2 x 1 blocks, 3 slots, 72 KB
+      if constexpr (EPI == EPI_STORE && !TNL)
+        return launch_ring_cfg<EPI, TNL, RingCfg<2, 2, 2, 1, 3>>(g, rows, cols, batch, stream, what);
+      [[fallthrough]];    // (the symmetric products take square tiles)
+    case RING_128_DEEP:   // 2 x 2 waves of 2 x 2 blocks, 4 slots, 128 KB
+      return launch_ring_cfg<EPI, TNL, RingCfg<2, 2, 2, 2, 4>>(g, rows, cols, batch, stream, what);
+    default:              // ... 2 slots, 64 KB
+      return launch_ring_cfg<EPI, TNL, RingCfg<2, 2, 2, 2, 2>>(g, rows, cols, batch, stream, what);
+  }
+}
+
 // Output tile size of the three phases (K1, K2, K3) for a shape.  Chosen from the
 // shape alone, never from the batch, so a matrix's result does not depend on the
 // batch it is computed in (the tile fixes each output's K-walk order).  The m x m
@@ -974,6 +1329,59 @@ static void phase_tiles(const ChainDims& d, int tile[3]) {
     for (int i = 0; i < 3; ++i) tile[i] = t[i] == 128 ? 128 : 256;
 }
 
+// gemm_ring configuration of each phase, or RING_NONE for gemm_nt_bf16 (all give the same
+// bits, so the batch may decide).  By the 64 x 64 tiles a phase has (ts of the symmetric
+// products, tt of T B'), from the chain's time with one phase changed at a time (us per
+// launch against RING_64; one box):
+//   K1  ts  420: 128_DEEP +7.6, NONE +68      630: 0 / +15     840: -20 / +37
+//       ts 1250: 128_DEEP  0, NONE  -9 (m <= 768)   1630: 128 -25, NONE -12 (m = 1024)
+//   K2  ts  840: 128_DEEP -2, NONE +16        936: -1 / +1    1680: 0 / +1   2500: +2 / 0
+//   K3  tt  432: 128x64 0, NONE +13           864: -2 / +8   1200: -0.6 / +8
+//       tt 1600: 128x64 -3, 128 -7, NONE -3  2304: -3 / -2 / -7
+// and for K3 of 3200 tiles or more NONE is ahead of every ring.  A width just past a
+// multiple of 256 costs gemm_nt_bf16 the padding: from 1.75 times the rings' products on
+// (m = 320, 520, 576; 96 x (576, 576) 1242 -> 932 us) they keep the larger batches too;
+// at 1.5 to 1.74 (m = 448, 833, 1100) it is as fast or faster.
+static void chain_cfg(const ChainDims& d, int batch, int cfg[3]) {
+  const long long tn = ceil_div(d.n, CHAIN_BLK), tm = ceil_div(d.m, CHAIN_BLK);
+  const long long ts = batch * (tm * (tm + 1) / 2), tt = batch * tn * tm;
+  const bool wide = d.mp > 768;
+  cfg[0] = ts <= 500 ? RING_64 : ts <= 1000 ? RING_128_DEEP : wide && ts <= 1700 ? RING_128 : RING_NONE;
+  cfg[1] = ts <= 1000 ? RING_64 : wide && ts <= 1700 ? RING_128_DEEP : RING_NONE;
+  cfg[2] = tt <= 448 ? RING_64 : tt <= 1400 ? RING_128x64 : tt <= 2000 ? RING_128 : RING_NONE;
+  // 64 x 64 x 64 products per matrix of either kernel
+  int tl[3];
+  phase_tiles(d, tl);
+  const long long pn = d.np / CHAIN_BLK, pm = d.mp / CHAIN_BLK;
+  auto sym = [&](int t) {   // upper tiles of an mp x mp product, in 64 x 64 units
+    const long long k = d.mp / t, u = t / CHAIN_BLK;
+    return k * (k + 1) / 2 * u * u;
+  };
+  const long long big = sym(tl[0]) * pn + sym(tl[1]) * pm + pn * pm * pm;
+  const long long ring = tm * (tm + 1) / 2 * (tn + tm) + tn * tm * tm;
+  if (4 * big >= 7 * ring) {
+    if (cfg[0] == RING_NONE) cfg[0] = RING_64;
+    if (cfg[1] == RING_NONE) cfg[1] = RING_64;
+    if (cfg[2] == RING_NONE) cfg[2] = RING_128;
+  }
+  if (getenv("DMH_CHAIN_TILES")) cfg[0] = cfg[1] = cfg[2] = RING_NONE;   // (names its tiles)
+  const char* env = getenv("DMH_CHAIN_RING");   // tuning override "k1_k2_k3"
+  int c[3];
+  if (env && sscanf(env, "%d_%d_%d", &c[0], &c[1], &c[2]) == 3)
+    for (int i = 0; i < 3; ++i) cfg[i] = c[i] >= RING_NONE && c[i] <= RING_128 ? c[i] : RING_NONE;
+}
+
+// with every phase on gemm_ring nothing past the last 64 x 64 block is read
+static bool all_ring(const int cfg[3]) { return cfg[0] && cfg[1] && cfg[2]; }
+
+void chain_extent(const ChainDims& d, int batch, int* rows, int* cols) {
+  int cfg[3];
+  chain_cfg(d, batch, cfg);
+  const bool ring = all_ring(cfg);
+  *rows = ring ? ceil_div(d.n, CHAIN_BLK) * CHAIN_BLK : d.np;
+  *cols = ring ? ceil_div(d.m, CHAIN_BLK) * CHAIN_BLK : d.mp;
+}
+
 int chain_run_packed(hipStream_t stream, const ChainWs& w, int batch, const ChainDims& d,
                      int orient_tall, const double* coeffs, int steps, bf16* outp) {
   if (steps == 0) {
@@ -986,6 +1394,9 @@ int chain_run_packed(hipStream_t stream, const ChainWs& w, int batch, const Chai
   }
   int tl[3];
   phase_tiles(d, tl);
+  int cfg[3], nc, mc;
+  chain_cfg(d, batch, cfg);
+  chain_extent(d, batch, &nc, &mc);
   // Consecutive launches walk the batch in opposite directions, so each one starts
   // on the matrices the previous one wrote last, which are still in the memory-side
   // cache (the group's operands are several times its size).  The entry pack wrote
@@ -1010,7 +1421,10 @@ int chain_run_packed(hipStream_t stream, const ChainWs& w, int batch, const Chai
     g1.valid_i = d.mp; g1.valid_j = d.mp;
     g1.rev = rev; rev ^= 1;
     g1.kspread = 1;
-    if ((rc = launch_gemm<EPI_STORE, 1>(g1, tl[0], d.mp, d.mp, batch, stream, "ns K1 (T^T T)")))
+    g1.kvalid = d.n; g1.ref_tile = tl[0];
+    if ((rc = cfg[0] ? launch_ring<EPI_STORE, 1>(g1, cfg[0], mc, mc, batch, stream, "ns K1 (T^T T)")
+                    : launch_gemm<EPI_STORE, 1>(g1, tl[0], d.mp, d.mp, batch, stream,
+                                                "ns K1 (T^T T)")))
       return rc;
     // K2: B = b A + c A A
     GemmArgs g2 = g1;
@@ -1022,8 +1436,11 @@ int chain_run_packed(hipStream_t stream, const ChainWs& w, int batch, const Chai
     g2.out = Bm; g2.outT = Bm;
     g2.rev = rev; rev ^= 1;
     g2.kspread = 0;
-    if ((rc = launch_gemm<EPI_POLY, 0>(g2, tl[1], d.mp, d.mp, batch, stream,
-                                      "ns K2 (bA + cA^2 + aI)")))
+    g2.kvalid = d.m; g2.ref_tile = tl[1];
+    if ((rc = cfg[1] ? launch_ring<EPI_POLY, 0>(g2, cfg[1], mc, mc, batch, stream,
+                                                 "ns K2 (bA + cA^2 + aI)")
+                    : launch_gemm<EPI_POLY, 0>(g2, tl[1], d.mp, d.mp, batch, stream,
+                                               "ns K2 (bA + cA^2 + aI)")))
       return rc;
     // K3: T' = T B' (the final iterate in the caller's orientation)
     GemmArgs g3{};
@@ -1042,7 +1459,10 @@ int chain_run_packed(hipStream_t stream, const ChainWs& w, int batch, const Chai
     }
     g3.rev = rev; rev ^= 1;
     g3.kspread = 2;
-    if ((rc = launch_gemm<EPI_STORE, 0>(g3, tl[2], d.np, d.mp, batch, stream, "ns K3 (T B')")))
+    g3.kvalid = d.m; g3.ref_tile = tl[2];
+    if ((rc = cfg[2] ? launch_ring<EPI_STORE, 0>(g3, cfg[2], nc, mc, batch, stream, "ns K3 (T B')")
+                    : launch_gemm<EPI_STORE, 0>(g3, tl[2], d.np, d.mp, batch, stream,
+                                                "ns K3 (T B')")))
       return rc;
     bf16* t = Tc; Tc = Tn; Tn = t;
   }
@@ -1093,7 +1513,9 @@ int dmh_ns_chain(hipStream_t stream, const void* x, int x_dtype, int batch, int 
                        w.partials);
     DMH_CHECK_LAUNCH("entry_norm_partials");
   }
-  hipLaunchKernelGGL(entry_pack, dim3(d.mp / 64, d.np / 64, batch), dim3(256), 0, stream, v,
+  int er, ec;
+  chain_extent(d, batch, &er, &ec);
+  hipLaunchKernelGGL(entry_pack, dim3(ec / 64, er / 64, batch), dim3(256), 0, stream, v,
                      orient_tall, entry_mode, w.partials, d.n, d.m, d.np, d.mp, w.T0);
   DMH_CHECK_LAUNCH("entry_pack");
   return chain_run_packed(stream, w, batch, d, orient_tall, coeffs, steps, (bf16*)out);

@@ -2641,7 +2641,8 @@ static int rsvd_core(hipStream_t st, const float* A, const float* Omega, int B, 
 static int launch_restore(hipStream_t st, const float* A, int B, int n, int m, const RsvdWs& w,
                           float* d, void* X0, int x0_mode, bf16* T, bf16* W, int np,
                           int mp) {
-  const int rows = T ? np : n, cols = T ? mp : m;
+  int rows = n, cols = m;
+  if (T) chain_extent(chain_dims(n, m, 1), B, &rows, &cols);
   hipLaunchKernelGGL(w_norm_partials, dim3(wn_parts(n, m), 1, B),
                      dim3(256), 0, st, A, n, m, w.U, w.V, w.kint, w.cw, w.wflag, w.wpart);
   DMH_CHECK_LAUNCH("w_norm_partials");

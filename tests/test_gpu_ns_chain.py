@@ -77,6 +77,38 @@ def test_tile_sizes_agree(N, shape, monkeypatch):
         assert rel(outs[tiles], outs[TILE_CHOICES[0]]) < 6e-2, tiles
 
 
+@pytest.mark.parametrize("ring", ["1_1_1", "1_1_2", "3_3_3", "4_4_4", "3_0_1", "0_1_4"])
+@pytest.mark.parametrize("shape", [(1, 64, 64), (2, 65, 33), (1, 192, 96), (3, 100, 300),
+                                   (1, 1000, 333), (2, 640, 320), (1, 1280, 1280), (1, 2111, 769)])
+def test_ring_gemm_matches_the_persistent_gemm(N, shape, ring, monkeypatch):
+    """The small-tile ring kernels sum every output's products in the persistent kernel's
+    order, so the chain comes out bit for bit the same in every configuration (K walks
+    shorter and longer than the ring, starts other than 0, ragged edges, phases mixed),
+    in both orientations."""
+    g = torch.Generator(device=DEV).manual_seed(sum(shape))
+    X = torch.randn(*shape, generator=g, device=DEV)
+    for tall in (True, False):
+        monkeypatch.setenv("DMH_CHAIN_RING", "0_0_0")
+        want = N.ns_chain(X, tall, 1, O.ns_schedule(3))
+        monkeypatch.setenv("DMH_CHAIN_RING", ring)
+        got = N.ns_chain(X, tall, 1, O.ns_schedule(3))
+        assert torch.isfinite(want.float()).all()
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), tall
+
+
+@pytest.mark.parametrize("m", [96, 333, 640])
+def test_chain_result_does_not_depend_on_the_batch(N, m):
+    """A matrix's polar factor is the same alone (ring kernels) and in batches that the
+    rule gives to other kernels."""
+    X = torch.randn(300, 2 * m, m, generator=torch.Generator(device=DEV).manual_seed(m),
+                    device=DEV)
+    one = [N.ns_chain(X[b:b + 1], True, 1, O.ns_schedule(5)) for b in (0, 7)]
+    for batch in (8, 24, 96, 300):
+        many = N.ns_chain(X[:batch], True, 1, O.ns_schedule(5))
+        for b, u in zip((0, 7), one):
+            assert torch.equal(many[b].view(torch.int16), u[0].view(torch.int16)), (batch, b)
+
+
 def test_zero_steps_and_entry(N):
     G = torch.randn(2, 96, 160, generator=torch.Generator().manual_seed(3))
     for mode, scale in ((1, 1.0), (2, 1.01)):
