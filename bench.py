@@ -416,10 +416,11 @@ def kernels_report(args, dev):
 
 def horner_f32_report(args, dev):
     """--mode horner-f32: the fp32 iteration (`_horner_iterate` on fp32 input, the
-    path the reference's convergence study runs; dmh_horner_f32 on the fp32 matrix
-    cores) over the workload's shape groups, 5 NS steps per matrix, the groups one
-    after the other on the launch stream; `args.steps` timed rounds after
-    `args.warmup`.  FLOP: the canonical 4m^2n + 2m^3 per matrix and step."""
+    path the reference's convergence study runs; dmh_horner_f32, six bf16 MFMA products
+    per fp32 product) over the workload's shape groups, 5 NS steps per matrix, the groups
+    one after the other on the launch stream; `args.steps` timed rounds after
+    `args.warmup`.  FLOP: the canonical 4m^2n + 2m^3 per matrix and step; the peak of
+    `frac_split_peak` is a sixth of the bf16 peak."""
     import torch
     from defmuon_amd.optim import deflation_batched as DB
     groups = WORKLOADS[args.workload]
@@ -448,7 +449,8 @@ def horner_f32_report(args, dev):
     log(f"bench horner-f32: {args.warmup} + {args.steps} rounds over {groups}")
     return {"mode": "horner-f32", "workload": args.workload, "groups": groups,
             "ms_per_step": round(ms, 3), "flop_per_step": flop, "tflops": round(tflops, 1),
-            "frac_fp32_mfma_peak": round(tflops / 157.3, 3), "steps": args.steps,
+            "frac_fp32_mfma_peak": round(tflops / 157.3, 3),
+            "frac_split_peak": round(tflops * 6 / PEAK_BF16_TFLOPS, 3), "steps": args.steps,
             "warmup": args.warmup}
 
 

@@ -205,3 +205,28 @@ def test_horner_fp32_keeps_dtype(N, shape, sched):
     assert rel(got2, want[0]) <= 1e-5
     with pytest.raises(N.NativeError):
         DB._horner_iterate(X.to(DEV).half(), hs)
+
+
+@pytest.mark.parametrize("sched", ["ns", "pe"])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 40, 32), (1, 127, 129), (3, 128, 96), (2, 333, 100),
+                                   (1, 1000, 333), (4, 1536, 768), (1, 2049, 513)])
+def test_horner_fp32_split_is_as_accurate_as_fp32(N, shape, sched, monkeypatch):
+    """fp32 input on the split-bf16 products: the error against 64 bits is within the 1e-5
+    the fp32 chain is held to, and no larger than that of the fp32 matrix cores on the same
+    input.  Each of the five steps rounds its result to fp32 (2^-24 relative) on either
+    path, so 5 * 2^-24 is what two correct evaluations of a single entry (shape (1, 1, 1))
+    may differ by; a tenth for the scatter of the longer sums."""
+    g = torch.Generator(device=DEV).manual_seed(sum(shape))
+    X = torch.randn(*shape, generator=g, device=DEV)
+    X = X / X.flatten(1).norm(dim=1)[:, None, None]
+    hs = O.ns_schedule(5) if sched == "ns" else O.pe_schedule(5)
+    want = X.double()
+    for a, b, c in hs:
+        Gm = want.mT.contiguous() @ want
+        want = a * want + want @ (b * Gm + c * (Gm @ Gm))
+    errs = {}
+    for split in "01":
+        monkeypatch.setenv("DMH_HORNER_SPLIT", split)
+        errs[split] = rel(N.horner_f32(X, hs), want)
+    assert errs["1"] < 1e-5, errs
+    assert errs["1"] <= 1.1 * errs["0"] + 5 * 2.0 ** -24, errs
