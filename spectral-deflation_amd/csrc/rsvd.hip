@@ -1532,15 +1532,13 @@ __global__ __launch_bounds__(EG_THREADS) void eig_gate(const double* __restrict_
 // eigenpairs (the deflated directions) and the eigenvalues the gate compares are
 // needed; one 512-thread workgroup per matrix.
 //  1. Householder reduction of H = Bp Bp^T (r x r, fp64) to tridiagonal form
-//     T = Q^T H Q (LAPACK's convention: reflector k = I - tau_k v_k v_k^T acts on
-//     rows k+1.., v_k[k+1] = 1, T[k+1][k] = ||H[k+1:, k]||), by one wave: lane l owns
-//     column l of the trailing block, kept whole (both triangles) in LDS, so every
-//     access is a row read or write across the lanes.
-//  2. Every eigenvalue of T by multisection: lane j of each of the 8 waves evaluates
-//     the Sturm count (the number of eigenvalues below x, from the pivots of
-//     T - x I) at one of 8 interior points of the j-th smallest eigenvalue's bracket,
-//     so each pass shrinks every bracket 9x (EH_PASSES passes from the Gershgorin
-//     interval).
+//     T = Q^T H Q (reflector k = I - tau_k v_k v_k^T acts on rows k+1..), H's rows in the
+//     waves' registers.
+//  2. The top kw eigenvalues of T by multisection: 16 (or 8) lanes per eigenvalue evaluate
+//     the Sturm count (the number of eigenvalues below x, from the leading minors of
+//     T - x I) at that many interior points of its bracket, so each pass shrinks every
+//     bracket 17x (9x); the points of a bracket are neighbouring lanes, so a ballot finds
+//     its next bounds and no pass needs a barrier.
 //  3. The top nv = min(kw, r) eigenpairs -- every value the gate compares at the
 //     default thresholds -- by inverse iteration on T (partial-pivoting elimination of
 //     T - sigma I, one lane per eigenpair, start vectors fixed per index, Rayleigh-
@@ -1548,7 +1546,11 @@ __global__ __launch_bounds__(EG_THREADS) void eig_gate(const double* __restrict_
 //     one re-orthogonalised in order after every step; further deflated directions
 //     the gate asks for (thresholds set apart) the same way afterwards.  Then each
 //     vector is back-transformed, Q y.
-//  4. The gate, the deflate / restore weights and d exactly as eig_gate computes them.
+//  4. The gate, the deflate / restore weights and d as eig_gate computes them.
+// Every phase is a chain of dependent fp64 operations of one workgroup.  us per launch at
+// r = 18 / 40 / 52 (6, 1 and 24 matrices): 51 / 87 / 112; with square roots and divisions in
+// the reflectors, Sturm ratios with a reciprocal per row, every loop over all 64 rows and d
+// on one wave: 91 / 134 / 161.
 // Degenerate matrices (flagged by the Cholesky) skip 1-3 and come out declined, as
 // in eig_gate.
 // ---------------------------------------------------------------------------
@@ -1560,11 +1562,13 @@ constexpr int ZP = RP + 2;      // row pitch (doubles) of the eigenvector rows
 
 union EhScratch {
   struct {
-    double H[RP * JP];                                 // H, reduced in place
+    double H[RP * JP];                                 // H as loaded
+    double row[2][RP];                                 // row k of the reduced H (by parity of k)
     double pw[EH_WAVES][RP];                           // the waves' partial products
   } red;                                               // (step 1)
   struct {
-    double u0[RP][EH_VL], u1[RP][EH_VL], u2[RP][EH_VL];   // band U of T - sigma I, per lane
+    // band U of T - sigma I, per lane (u0: the reciprocals of its diagonal)
+    double u0[RP][EH_VL], u1[RP][EH_VL], u2[RP][EH_VL];
     double y[RP][EH_VL];                                  // the lane's vector
   } lu;                                                // (step 4)
   double G[RP * JP];                                   // Q^T Q (step 5)
@@ -1609,11 +1613,6 @@ __device__ __forceinline__ double wave_max_d(double v) {
   v = fmax(v, dpp_d(v, 3));
   return fmax(fmax(lane_val(v, 0), lane_val(v, 16)), fmax(lane_val(v, 32), lane_val(v, 48)));
 }
-// 1/x from the hardware estimate and one Newton step
-__device__ __forceinline__ double rcp_nr1(double x) {
-  double y = __builtin_amdgcn_rcp(x);
-  return fma(y, fma(-x, y, 1.0), y);
-}
 // the compiler keeps LDS accesses on either side in order; a wave's LDS accesses
 // complete in order, so reads after it see every lane's earlier writes
 __device__ __forceinline__ void wave_lds_order() {
@@ -1646,6 +1645,8 @@ __device__ __forceinline__ void eh_inverse_iteration(int t0, int t1, int r, doub
   const int cl = lane ? l : 0;
   const double eps_tn = 2.220446049250313e-16 * (tn > 0.0 ? tn : 1.0);
   double sigma = act ? lamd[t] : 0.0;
+  // rows to walk: past r the vectors are zero and T is decoupled
+  const int rr = min(RP, (r + 7) & ~7);
   if (lane) {
     double n0 = 0.0;
     for (int i = 0; i < RP; ++i) {
@@ -1654,7 +1655,7 @@ __device__ __forceinline__ void eh_inverse_iteration(int t0, int t1, int r, doub
       sc.lu.y[i][cl] = v;
     }
     const double s0n = n0 > 0.0 ? rsqrt_nr(n0) : 0.0;
-    for (int i = 0; i < RP; ++i) sc.lu.y[i][cl] *= s0n;
+    for (int i = 0; i < rr; ++i) sc.lu.y[i][cl] *= s0n;
   }
   // a step has converged when the solve amplified the unit start vector by 1e8 / ||T||
   // (the shift then lies within ~1e-8 ||T|| |c| of the eigenvalue, c the start vector's
@@ -1666,13 +1667,14 @@ __device__ __forceinline__ void eh_inverse_iteration(int t0, int t1, int r, doub
       double cur0 = dd[0] - sigma, cur1 = ee[0];
       double yc = sc.lu.y[0][cl];
 #pragma unroll 4
-      for (int i = 0; i + 1 < RP; ++i) {
+      for (int i = 0; i + 1 < rr; ++i) {
         const double sub = ee[i], nd = dd[i + 1] - sigma, ns = (i + 2 < RP) ? ee[i + 1] : 0.0;
         const double yn = sc.lu.y[i + 1][cl];
         const bool sw = fabs(cur0) < fabs(sub);
         const double piv = sw ? sub : (cur0 != 0.0 ? cur0 : eps_tn);
-        const double mlt = (sw ? cur0 : sub) * rcp_nr(piv);
-        sc.lu.u0[i][cl] = piv;
+        const double ipiv = rcp_nr(piv);
+        const double mlt = (sw ? cur0 : sub) * ipiv;
+        sc.lu.u0[i][cl] = ipiv;
         sc.lu.u1[i][cl] = sw ? nd : cur1;
         sc.lu.u2[i][cl] = sw ? ns : 0.0;
         sc.lu.y[i][cl] = sw ? yn : yc;
@@ -1681,15 +1683,17 @@ __device__ __forceinline__ void eh_inverse_iteration(int t0, int t1, int r, doub
         cur1 = sw ? -mlt * ns : ns;
         cur0 = c0;
       }
-      sc.lu.u0[RP - 1][cl] = cur0 != 0.0 ? cur0 : eps_tn;
+      sc.lu.u0[rr - 1][cl] = rcp_nr(cur0 != 0.0 ? cur0 : eps_tn);
+      sc.lu.u1[rr - 1][cl] = 0.0;
+      sc.lu.u2[rr - 1][cl] = 0.0;
       // back substitution, then |x| and the Rayleigh quotient
       double x1 = 0.0, x2 = 0.0, nrm = 0.0;
 #pragma unroll 4
-      for (int i = RP - 1; i >= 0; --i) {
-        const double yi = i == RP - 1 ? yc : sc.lu.y[i][cl];
+      for (int i = rr - 1; i >= 0; --i) {
+        const double yi = i == rr - 1 ? yc : sc.lu.y[i][cl];
         double s = fma(-sc.lu.u1[i][cl], x1, yi);
         s = fma(-sc.lu.u2[i][cl], x2, s);
-        const double x = s * rcp_nr(sc.lu.u0[i][cl]);
+        const double x = s * sc.lu.u0[i][cl];
         sc.lu.y[i][cl] = x;
         nrm = fma(x, x, nrm);
         x2 = x1;
@@ -1699,7 +1703,7 @@ __device__ __forceinline__ void eh_inverse_iteration(int t0, int t1, int r, doub
       conv = nrm * tn * tn >= 1e16;
       double rq = 0.0, rq2 = 0.0, yp = 0.0;
 #pragma unroll 8
-      for (int i = 0; i < RP; ++i) {
+      for (int i = 0; i < rr; ++i) {
         const double yi = sc.lu.y[i][cl] * inv;
         sc.lu.y[i][cl] = yi;
         rq = fma(dd[i] * yi, yi, rq);
@@ -1739,7 +1743,7 @@ __device__ __forceinline__ void eh_inverse_iteration(int t0, int t1, int r, doub
   if (act) {
     double rq = 0.0, rq2 = 0.0, yp = 0.0;
 #pragma unroll 8
-    for (int i = 0; i < RP; ++i) {
+    for (int i = 0; i < rr; ++i) {
       const double yi = sc.lu.y[i][cl];
       rq = fma(dd[i] * yi, yi, rq);
       if (i > 0) rq2 = fma(ee[i - 1] * yp, yi, rq2);
@@ -1802,8 +1806,7 @@ __global__ __launch_bounds__(EH_THREADS) void eig_head_gate(
   __shared__ __attribute__((aligned(16))) EhScratch sc;
   __shared__ __attribute__((aligned(16))) double Vr[RP * RP];   // reflector k in row k
   __shared__ __attribute__((aligned(16))) double Z[RP * ZP];    // eigenvector t in row t
-  __shared__ double dd[RP], ee[RP], e2s[RP], taus[RP], lamd[RP];
-  __shared__ int cnt[2][EH_THREADS];
+  __shared__ double dd[RP], ee[RP], ds[RP], e2s[RP], taus[RP], lamd[RP];
   __shared__ float sv[RP];
   __shared__ double s_lo, s_hi, s_tn;
   const int b = blockIdx.x, tid = threadIdx.x, l = tid & 63;
@@ -1821,70 +1824,93 @@ __global__ __launch_bounds__(EH_THREADS) void eig_head_gate(
     }
   }
   __syncthreads();
-  // ---- 1. tridiagonal reduction: every wave forms each reflector itself (the same
-  // values: same inputs, same order), so that only the matrix-vector product and the
-  // rank-2 update, whose rows (every 8th) the waves share, need workgroup barriers
+  // ---- 1. tridiagonal reduction.  Wave w keeps rows w, w + 8, ... of H in registers (lane
+  // l: column l); row k goes through LDS to every wave, and each forms reflector k itself
+  // (the same values: same inputs, same order), so that only the matrix-vector product and
+  // the published row need workgroup barriers.  Reflector k is I - tau v v^T with
+  // v = x + sign(x_0) |x| e_1 for x = H[k+1:, k], tau = 1 / (|x|^2 + |x_0| |x|): one reciprocal
+  // square root and one reciprocal in the chain, and entries of v and w up to k are zero, so
+  // the product and the update run over all rows and columns without conditions.
+  // (r = 64: 64 us per workgroup; 90 with H in LDS and a square root and divisions.)
   if (!bad) {
     double* H = sc.red.H;
+    double h[RP / EH_WAVES];
+#pragma unroll
+    for (int q = 0; q < RP / EH_WAVES; ++q) h[q] = H[(wave + EH_WAVES * q) * JP + l];
+    if (wave == 0) sc.red.row[0][l] = h[0];
+    __syncthreads();
     for (int k = 0; k + 2 < r; ++k) {
-      const double xi = (l > k && l < r) ? H[k * JP + l] : 0.0;   // H[l][k] = H[k][l]
+      const double rk = sc.red.row[k & 1][l];   // H[k][l]
+      const double xi = (l > k && l < r) ? rk : 0.0;
       const double x0 = lane_val(xi, k + 1);
       const double sg = wave_sum_d(l > k + 1 ? xi * xi : 0.0);
       double vl = 0.0, tk = 0.0, ek = x0;   // sg == 0: already reduced, no reflection
       if (sg != 0.0) {
-        const double mu = sqrt(x0 * x0 + sg);
-        const double v0 = x0 <= 0.0 ? x0 - mu : -sg / (x0 + mu);
-        const double v02 = v0 * v0;
-        tk = 2.0 * v02 / (sg + v02);
-        const double iv0 = 1.0 / v0;
-        vl = l == k + 1 ? 1.0 : ((l > k + 1 && l < r) ? xi * iv0 : 0.0);
-        ek = mu;
+        const double s2 = fma(x0, x0, sg);
+        const double mu = s2 * rsqrt_nr(s2);
+        vl = l == k + 1 ? x0 + copysign(mu, x0) : xi;
+        ek = -copysign(mu, x0);
+        tk = rcp_nr(fma(fabs(x0), mu, s2));
       }
       if (wave == 0) {
         Vr[k * RP + l] = vl;
-        if (l == 0) { dd[k] = H[k * JP + k]; ee[k] = ek; taus[k] = tk; }
+        if (l == k) { dd[k] = rk; ee[k] = ek; taus[k] = tk; }
       }
       if (tk != 0.0) {   // uniform over the workgroup
-        // p = tau H22 v: wave w sums rows k+1+w, k+1+w+8, ... (lane l: column l)
-        double a0 = 0.0, a1 = 0.0;
-        int j = k + 1 + wave;
-        for (; j + EH_WAVES < r; j += 2 * EH_WAVES) {
-          a0 = fma(H[j * JP + l], lane_val(vl, j), a0);
-          a1 = fma(H[(j + EH_WAVES) * JP + l], lane_val(vl, j + EH_WAVES), a1);
+        double vj[RP / EH_WAVES], a0 = 0.0, a1 = 0.0;
+#pragma unroll
+        for (int q = 0; q < RP / EH_WAVES; q += 2) {
+          vj[q] = lane_val(vl, wave + EH_WAVES * q);
+          vj[q + 1] = lane_val(vl, wave + EH_WAVES * (q + 1));
+          a0 = fma(h[q], vj[q], a0);
+          a1 = fma(h[q + 1], vj[q + 1], a1);
         }
-        if (j < r) a0 = fma(H[j * JP + l], lane_val(vl, j), a0);
         sc.red.pw[wave][l] = a0 + a1;
         __syncthreads();
-        double pl = 0.0;
+        double p[EH_WAVES];
 #pragma unroll
-        for (int w = 0; w < EH_WAVES; ++w) pl += sc.red.pw[w][l];   // same order in every wave
+        for (int w = 0; w < EH_WAVES; ++w) p[w] = sc.red.pw[w][l];   // same order in every wave
+        double pl = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
         pl = (l > k && l < r) ? tk * pl : 0.0;
         const double K = wave_sum_d(pl * vl);
-        const double wl = pl - (0.5 * tk * K) * vl;
-        // H22 -= v w^T + w v^T, rows k+1+w, k+1+w+8, ... by wave w
-        for (int jj = k + 1 + wave; jj < r; jj += EH_WAVES) {
-          const double vj = lane_val(vl, jj), wj = lane_val(wl, jj);
-          if (l > k && l < r) {
-            double h = H[jj * JP + l];
-            h = fma(-vj, wl, h);
-            h = fma(-wj, vl, h);
-            H[jj * JP + l] = h;
-          }
+        const double wl = fma(-0.5 * tk * K, vl, pl);
+        // H22 -= v w^T + w v^T
+#pragma unroll
+        for (int q = 0; q < RP / EH_WAVES; ++q) {
+          const double wj = lane_val(wl, wave + EH_WAVES * q);
+          h[q] = fma(-vj[q], wl, h[q]);
+          h[q] = fma(-wj, vl, h[q]);
         }
+      }
+      if (wave == ((k + 1) & (EH_WAVES - 1))) {
+        double hr = h[0];
+#pragma unroll
+        for (int q = 1; q < RP / EH_WAVES; ++q) hr = q == (k + 1) / EH_WAVES ? h[q] : hr;
+        sc.red.row[(k + 1) & 1][l] = hr;
       }
       __syncthreads();
     }
+    // the trailing 2 x 2 block: row r - 2 was published by the last step (row 0 when r <= 2),
+    // row r - 1 by its owner now
+    static_assert(EH_WAVES == 8, "rows by wave");
+    if (r >= 2 && wave == ((r - 1) & (EH_WAVES - 1))) {
+      double hr = h[0];
+#pragma unroll
+      for (int q = 1; q < RP / EH_WAVES; ++q) hr = q == (r - 1) / EH_WAVES ? h[q] : hr;
+      sc.red.row[(r - 1) & 1][l] = hr;
+    }
+    __syncthreads();
     if (wave == 0) {
       // the trailing 2 x 2 (or 1 x 1) block; padding past r: a diagonal far above the
       // spectrum, decoupled (zero off-diagonal), so it never counts and never mixes in
       if (l == 0) {
         if (r >= 2) {
-          dd[r - 2] = H[(r - 2) * JP + r - 2];
-          dd[r - 1] = H[(r - 1) * JP + r - 1];
-          ee[r - 2] = H[(r - 1) * JP + r - 2];
+          dd[r - 2] = sc.red.row[r & 1][r - 2];
+          dd[r - 1] = sc.red.row[(r - 1) & 1][r - 1];
+          ee[r - 2] = sc.red.row[(r - 1) & 1][r - 2];
           taus[r - 2] = 0.0;
         } else {
-          dd[0] = H[0];
+          dd[0] = sc.red.row[0][0];
         }
       }
       wave_lds_order();
@@ -1899,8 +1925,6 @@ __global__ __launch_bounds__(EH_THREADS) void eig_head_gate(
       if (l >= r) dd[l] = 2.0 * tn + 1.0;
       if (l + 1 >= r) ee[l] = 0.0;
       if (l + 2 >= r && l < r) taus[l] = 0.0;
-      wave_lds_order();
-      e2s[l] = ee[l] * ee[l];
       if (l == 0) {   // brackets widened by rounding-level margins
         const double mg = 4.0 * 2.220446049250313e-16 * (tn * RP) + 1e-300;
         s_lo = lo - mg;
@@ -1918,42 +1942,58 @@ __global__ __launch_bounds__(EH_THREADS) void eig_head_gate(
   const int npt = nE <= 32 ? 16 : 8;           // points per bracket
   const int slot = tid / npt, pt = tid % npt;  // eigenvalue slot (descending), point
   if (!bad) {
-    double e2max = 0.0;
-    for (int i = 0; i + 1 < r; ++i) e2max = fmax(e2max, e2s[i]);
-    const double pivmin = 2.2250738585072014e-308 * fmax(1.0, e2max);
+    // T / ||T||: the Sturm counts below then need no care for the range of T
+    if (wave == 0) {
+      const double it = s_tn > 0.0 ? 1.0 / s_tn : 1.0;
+      // (1e-60: far below rounding, so that no coupling is exactly zero)
+      ds[l] = l < r ? dd[l] * it : 4.0;
+      const double em = l > 0 ? ee[l - 1] * it : 0.0;
+      e2s[l] = l > 0 ? fmax(em * em, 1e-60) : 0.0;
+    }
+    __syncthreads();
+    const double it = s_tn > 0.0 ? 1.0 / s_tn : 1.0;
     const int npass = npt == 16 ? 9 : 12;      // brackets ~2 ||T|| / 17^9 or / 9^12
     const double inv_sect = 1.0 / (double)(npt + 1);
     double L = s_lo, U = s_hi;
     const int j = r - 1 - slot;                // ascending index of the eigenvalue
     const bool live = slot < nE;
+    const int r8 = (r + 7) & ~7;               // (padding past r: far above, never counts)
     for (int p = 0; p < npass; ++p) {
-      // (the same expression as the readers' below, so all threads agree on the points)
       const double x = fma(U - L, (double)(pt + 1) * inv_sect, L);
       int c = 0;
       if (live) {
-        asm volatile("" ::: "memory");   // T's rows are read in batches, not all up front
-        double q = dd[0] - x;
-        if (fabs(q) < pivmin) q = -pivmin;
-        c = q < 0.0;
+        // Sturm count from the leading minors of T - x I, f_i = (d_i - x) f_{i-1} - e^2_{i-1}
+        // f_{i-2}: the number of sign changes, here of sign bits (one fma of latency per row,
+        // where the pivots' ratio form needs a reciprocal).  A minor that is zero keeps the
+        // total right whichever its sign bit, as the next one is -e^2 f_{i-2} (e^2 > 0).  Every
+        // 8 rows the last two are scaled by a power of two, so that they stay in range.
+        const double xs = x * it;
+        double f1 = 1.0, f2 = 0.0;
+        for (int i0 = 0; i0 < r8; i0 += 8) {
+          double dr[8], er[8];
 #pragma unroll
-        for (int i = 1; i < RP; ++i) {
-          if ((i & 7) == 0) asm volatile("" ::: "memory");
-          q = (dd[i] - x) - e2s[i - 1] * rcp_nr1(q);
-          if (fabs(q) < pivmin) q = -pivmin;
-          c += q < 0.0;
+          for (int i = 0; i < 8; ++i) {
+            dr[i] = ds[i0 + i] - xs;
+            er[i] = e2s[i0 + i];     // (e2s[i]: of rows i - 1 and i)
+          }
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const double f = fma(dr[i], f1, -(er[i] * f2));
+            c += (unsigned)(__double2hiint(f) ^ __double2hiint(f1)) >> 31;
+            f2 = f1;
+            f1 = f;
+          }
+          const int e = -__builtin_amdgcn_frexp_exp(fmax(fabs(f1), fabs(f2)));
+          f1 = ldexp(f1, e);
+          f2 = ldexp(f2, e);
         }
       }
-      cnt[p & 1][tid] = c;
-      __syncthreads();
-      double nL = L, nU = U;
-      bool found = false;
-      for (int w = 0; w < npt; ++w) {
-        const double xw = fma(U - L, (double)(w + 1) * inv_sect, L);
-        if (!found) {
-          if (cnt[p & 1][slot * npt + w] > j) { nU = xw; found = true; }
-          else nL = xw;
-        }
-      }
+      // the first point whose count passes j ends the bracket (a bracket's points are npt
+      // consecutive lanes of one wave)
+      const unsigned long long past = __ballot(c > j) >> (l & ~(npt - 1));
+      const int w0 = __ffsll((past & ((1ull << npt) - 1)) | (1ull << npt)) - 1;
+      const double nL = w0 > 0 ? fma(U - L, (double)w0 * inv_sect, L) : L;
+      const double nU = w0 < npt ? fma(U - L, (double)(w0 + 1) * inv_sect, L) : U;
       L = nL;
       U = nU;
     }
@@ -2027,26 +2067,32 @@ __global__ __launch_bounds__(EH_THREADS) void eig_head_gate(
     }
     __syncthreads();
   }
-  if (!d_out || wave != 0) return;
+  if (!d_out) return;
   // ||W||_F^2 = ||A||^2 - sum_{t<k} lambda_t (2 - G_t), G_t = Ub_t^T (Q^T Q) Ub_t (see
-  // eig_gate)
+  // eig_gate); G_t by wave t % 8, summed in order by the first
+  if (fired) {   // uniform over the workgroup
+    const double* G = sc.G;
+    for (int t = wave; t < kk; t += EH_WAVES) {
+      double y0 = 0.0, y1 = 0.0;   // (Q^T Q Ub_t)_l, with Ub_t rounded to fp32 as stored
+      const double zl = l < r ? (double)(float)Z[t * ZP + l] : 0.0;
+      for (int c = 0; c < RP; c += 2) {   // (G is symmetric: lane l reads column l; zero past r)
+        y0 = fma(G[c * JP + l], (double)(float)Z[t * ZP + c], y0);
+        y1 = fma(G[(c + 1) * JP + l], (double)(float)Z[t * ZP + c + 1], y1);
+      }
+      const double gt = wave_sum_d(zl * (y0 + y1));
+      if (l == 0) taus[t] = gt;   // (the reflectors are no longer needed)
+    }
+    __syncthreads();
+  }
+  if (wave != 0) return;
   double asum = 0.0;
   for (int i = l; i < asq_n; i += 64) asum += asq[(long long)b * asq_n + i];
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) asum += __shfl_xor(asum, o);
   double w2 = asum;
   if (fired) {
-    const double* G = sc.G;
     double head = 0.0;
-    for (int t = 0; t < kk; ++t) {
-      double y = 0.0;   // (Q^T Q Ub_t)_l, with Ub_t rounded to fp32 as stored
-      if (l < r)
-        for (int c = 0; c < r; ++c) y = fma(G[l * JP + c], (double)(float)Z[t * ZP + c], y);
-      double gt = (l < r) ? (double)(float)Z[t * ZP + l] * y : 0.0;
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) gt += __shfl_xor(gt, o);
-      head += lamd[t] * (2.0 - gt);
-    }
+    for (int t = 0; t < kk; ++t) head += lamd[t] * (2.0 - taus[t]);
     w2 = asum - head;
   }
   if (l == 0) d_out[b] = (float)sqrt(w2 > 0.0 ? w2 : 0.0) + 1e-7f;

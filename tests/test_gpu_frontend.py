@@ -378,3 +378,30 @@ def test_skinny_rows_direct_to_lds_matches_register_kernel(N, B, n, m, monkeypat
         assert torch.equal(a, b)
     assert float(((d - dr).abs() / dr).max()) < 1e-6
     assert rel(X0, X0r) < 1e-6
+
+
+@pytest.mark.parametrize("kind", ["spiked", "orthonormal", "axes"])
+@pytest.mark.parametrize("m", [1, 2, 3, 40, 41, 160, 161, 321, 1280])
+def test_clip_sketch_width_edges(N, m, kind):
+    """Sketch widths 1, 2, 4, 8, 10, 18 and 64 (the eigenproblem's row groups and their
+    remainders), on spectra that leave its tridiagonal form coupled, with one repeated value
+    everywhere, and with exact zeros off the diagonal, at three scales: gate, d and X0 as the
+    oracle's (1e-4, the subspace bound of the fp32 path)."""
+    from defmuon_amd import synthetic as S
+    n = 2 * m + 3
+    if kind == "spiked":
+        A = S.spiked_matrix(n, m, seed=m, n_spikes=1 if m >= 40 else 0, hi=50.0, lo=20.0)
+    elif kind == "orthonormal":
+        A = torch.linalg.qr(torch.randn(n, m, generator=torch.Generator().manual_seed(m)))[0]
+    else:
+        A = torch.zeros(n, m)
+        A[torch.arange(m), torch.arange(m)] = torch.where(torch.arange(m) < 1, 30.0, 1.0)
+    r, kw = O.sketch_dims(m)
+    Om = O.draw_omega(1, m, r, 7)
+    for scale in (1.0, 1e-6, 1e6):
+        As = (A * scale)[None].contiguous()
+        X0, k, d = N.rmfro_clip(As.to(DEV), Om.to(DEV), kw, 0.10, 0.10, 1.01)
+        X0o, ko, do = O.rmfro_clip(As, Om, out_dtype=torch.float32)
+        assert torch.equal(k.cpu(), ko), scale
+        assert torch.allclose(d.cpu(), do, rtol=1e-4), scale
+        assert rel(X0.cpu(), X0o) < 1e-4, scale
