@@ -31,6 +31,7 @@
 #include "ns_chain.h"
 
 #include <math.h>
+#include <stdlib.h>
 
 namespace dmh {
 
@@ -171,19 +172,20 @@ __device__ __forceinline__ double lane_val(double v, int lane) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-// 1/sqrt(x) and 1/x in fp64 from the hardware estimates plus Newton steps
-// (relative error ~1e-16 for the positive normal arguments used here)
+// 1/sqrt(x) and 1/x in fp64 from the hardware estimates y (relative error e ~ 2^-24) plus one
+// third-order step each: y (1 - e)^(-1/2) ~ y (1 + e / 2 + 3 e^2 / 8) with e = 1 - x y^2, and
+// y / (1 - e) ~ y (1 + e + e^2) with e = 1 - x y, both to e^3 ~ 2^-72: relative error ~1e-16 for
+// the positive normal arguments used here, in four and three dependent operations (two Newton
+// steps take eight and four)
 __device__ __forceinline__ double rsqrt_nr(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  y = y * (1.5 - 0.5 * x * y * y);
-  y = y * (1.5 - 0.5 * x * y * y);
-  return y;
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * y), y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
 }
 __device__ __forceinline__ double rcp_nr(double x) {
-  double y = __builtin_amdgcn_rcp(x);
-  y = y * (2.0 - x * y);
-  y = y * (2.0 - x * y);
-  return y;
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(y, fma(e, e, e), y);
 }
 
 // One workgroup per matrix.  Lane l of every wave keeps row l of the (identity-padded)
@@ -197,9 +199,10 @@ __device__ __forceinline__ double rcp_nr(double x) {
 // substitution.
 constexpr int CHOL_THREADS = 512;   // all sum the Gram partials and factor; wave 0 inverts
 
+// first: degen[b] is written (0 or 1); otherwise only raised
 __global__ __launch_bounds__(CHOL_THREADS) void chol_inv(const double* __restrict__ part, int r,
                                                          float* __restrict__ M,
-                                                         int* __restrict__ degen) {
+                                                         int* __restrict__ degen, int first) {
   constexpr int LP = RP + 2;   // row pitch (doubles): 16-byte aligned rows, 4-way at most
   constexpr int PER = RP * RP / CHOL_THREADS;
   const int b = blockIdx.x, tid = threadIdx.x, l = tid & 63;
@@ -231,7 +234,9 @@ __global__ __launch_bounds__(CHOL_THREADS) void chol_inv(const double* __restric
   // multipliers by readlane) and publishes them in rows CW p .. of Lc; after one barrier
   // the waves of later panels apply the CW new columns to theirs.  Every element sees
   // the same operations in the same order as in a one-wave loop over k (one barrier per
-  // panel instead of one per pivot: 25 -> 11 us per workgroup).
+  // panel instead of one per pivot: 25 -> 11 us per workgroup).  (The later waves'
+  // multipliers by readlane instead of broadcast LDS reads, here and in the inverse: 23 -> 28
+  // us per launch at r = 52.)
   constexpr int CW = RP / (CHOL_THREADS / 64);   // columns per wave
   static_assert(RP % (CHOL_THREADS / 64) == 0, "the waves share the columns evenly");
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -239,7 +244,9 @@ __global__ __launch_bounds__(CHOL_THREADS) void chol_inv(const double* __restric
 #pragma unroll
   for (int c = 0; c < CW; ++c) g[c] = Ls[l * LP + CW * wave + c];
   bool fail = false;
-  for (int pnl = 0; pnl < CHOL_THREADS / 64; ++pnl) {
+  // (past r the Gram is the identity: its panels need no factoring, and M is zero there)
+  const int npnl = (r + CW - 1) / CW;
+  for (int pnl = 0; pnl < npnl; ++pnl) {
     if (wave == pnl) {
 #pragma unroll
       for (int kc = 0; kc < CW; ++kc) {
@@ -257,7 +264,7 @@ __global__ __launch_bounds__(CHOL_THREADS) void chol_inv(const double* __restric
       }
     }
     __syncthreads();
-    if (wave > pnl) {
+    if (wave > pnl && wave < npnl) {
 #pragma unroll
       for (int kc = 0; kc < CW; ++kc) {
         const int k = CW * pnl + kc;
@@ -291,7 +298,7 @@ __global__ __launch_bounds__(CHOL_THREADS) void chol_inv(const double* __restric
     s1[q] = 0.0;
     xr[q] = 0.0;
   }
-  for (int J = 0; J < CHOL_THREADS / 64; ++J) {
+  for (int J = 0; J < npnl; ++J) {
     if (wave == J) {
 #pragma unroll
       for (int q = 0; q < CW; ++q) {
@@ -307,7 +314,7 @@ __global__ __launch_bounds__(CHOL_THREADS) void chol_inv(const double* __restric
       }
     }
     __syncthreads();
-    if (wave > J) {
+    if (wave > J && wave < npnl) {
 #pragma unroll
       for (int t2 = 0; t2 < CW; ++t2) {
         const int t = CW * J + t2;
@@ -334,7 +341,7 @@ __global__ __launch_bounds__(CHOL_THREADS) void chol_inv(const double* __restric
     v.w = (!fail && l < r && c + 3 < r) ? (float)xr[q + 3] : 0.f;
     *(float4*)&Mb[q] = v;
   }
-  if (tid == 0 && degen && fail) degen[b] = 1;
+  if (tid == 0 && (first || fail)) degen[b] = fail ? 1 : 0;
 }
 
 // C (rows x RP) = Y (rows x RP) * M (RP x RP), per matrix; 64 rows per workgroup,
@@ -655,6 +662,91 @@ __global__ __launch_bounds__(64) void gram_partials_pair(const float* __restrict
   else
     gram_chunk<S2>(Y2, rows2, (long long)rows2 * RP, part2, blockIdx.y,
                    blockIdx.x - GRAM_CHUNKS, threadIdx.x);
+}
+
+// The same partials with each chunk's rows over GRAM_WAVES waves, for batches whose chunks
+// leave most SIMDs without a wave: the waves' blocks are added in LDS in wave order.  One wave
+// per chunk walks its rows alone (one 3072-row panel: 30.5 us; 10 here).  us of a whole
+// front-end, one wave / four: 1 x (3072, 768) 398 / 335, 24 x (1024, 1024) 480 / 451, 48 x
+// (768, 768) 461 / 449, 72 x (5120, 1280) 2938 / 2906, 96 x (1024, 1024) 992 / 974, but 96 x
+// (1280, 320) 532 / 536, 144 x (1280, 1280) 1705 / 1733, 144 x (320, 320) 387 / 414.
+// Both operands in one launch when rows2 > 0: grid ((rows2 ? 2 : 1) GRAM_CHUNKS, batch).
+constexpr int GRAM_WAVES = 4;
+constexpr int GRAM_ACC = 40;   // doubles per lane: the ten blocks
+
+__global__ __launch_bounds__(64 * GRAM_WAVES) void gram_partials_mw(
+    const float* __restrict__ Y1, int rows1, double* __restrict__ part1,
+    const float* __restrict__ Y2, int rows2, double* __restrict__ part2) {
+  __shared__ __attribute__((aligned(16))) double sm[GRAM_WAVES * GRAM_ACC * 64];
+  const int b = blockIdx.y, tid = threadIdx.x, l = tid & 63, wave = tid >> 6;
+  const bool second = (int)blockIdx.x >= GRAM_CHUNKS;
+  const int chunk = second ? blockIdx.x - GRAM_CHUNKS : blockIdx.x;
+  const int rows = second ? rows2 : rows1;
+  const float* Y = (second ? Y2 : Y1) + (long long)b * rows * RP;
+  double* out = (second ? part2 : part1) + ((long long)b * GRAM_CHUNKS + chunk) * RP * RP;
+  const int per = (rows + GRAM_CHUNKS - 1) / GRAM_CHUNKS;
+  const int sub = ((per + GRAM_WAVES - 1) / GRAM_WAVES + 3) & ~3;   // whole 4-row MFMA steps
+  const int c0 = chunk * per, c1 = min(rows, c0 + per);
+  const int lo = min(c0 + wave * sub, c1), hi = min(lo + sub, c1);
+  const __amdgpu_buffer_rsrc_t yr = sk_rsrc(Y, (long long)rows * RP);
+  const int kr = l >> 4, cq = 4 * (l & 15);
+  auto load = [&](int r0, float4 (&v)[GRAM_G]) {
+#pragma unroll
+    for (int u = 0; u < GRAM_G; ++u) {
+      const int row = r0 + 4 * u + kr;
+      v[u] = sk_ld4(yr, row < hi ? (unsigned)(row * RP + cq) * 4u : SK_OOB);
+    }
+  };
+  f64x4 acc[10];
+#pragma unroll
+  for (int t = 0; t < 10; ++t) acc[t] = f64x4{0.0, 0.0, 0.0, 0.0};
+  constexpr int SET = 4 * GRAM_G;
+  float4 va[GRAM_G], vb[GRAM_G];
+  load(lo, va);
+  for (int r = lo; r < hi; r += 2 * SET) {   // (register sets in turn, as gram_chunk)
+    load(r + SET, vb);
+    asm volatile("" ::: "memory");
+    gram_mfma(va, acc);
+    asm volatile("" ::: "memory");
+    load(r + 2 * SET, va);
+    asm volatile("" ::: "memory");
+    gram_mfma(vb, acc);
+    asm volatile("" ::: "memory");
+  }
+#pragma unroll
+  for (int t = 0; t < 10; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sm[(wave * GRAM_ACC + 4 * t + e) * 64 + l] = acc[t][e];
+  __syncthreads();
+  // thread (wave, l) sums entries wave, wave + 4, ... of lane l's forty
+  double v[GRAM_ACC / GRAM_WAVES];
+#pragma unroll
+  for (int i = 0; i < GRAM_ACC / GRAM_WAVES; ++i) {
+    const int q = wave + GRAM_WAVES * i;
+    v[i] = sm[q * 64 + l];
+#pragma unroll
+    for (int w = 1; w < GRAM_WAVES; ++w) v[i] += sm[(w * GRAM_ACC + q) * 64 + l];
+  }
+  __syncthreads();
+  // the 64 x 64 partial through LDS as whole rows (as gram_chunk's short chunks): entry
+  // q = 4 t + e of lane l is block t = (c, c2), element e -- and wave = e
+  static_assert(GRAM_WAVES == 4, "a thread's entries share e");
+  {
+    int t = 0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int c2 = c; c2 < 4; ++c2, ++t) {
+        const int p = 4 * (kr + 4 * wave) + c, q = cq + c2;
+        sm[p * (RP + 2) + q] = v[t];
+        if (c != c2) sm[q * (RP + 2) + p] = v[t];
+      }
+  }
+  __syncthreads();
+  for (int i = tid; i < RP * RP / 2; i += 64 * GRAM_WAVES) {
+    const int row = i >> 5, col = 2 * (i & 31);
+    *(double2*)&out[row * RP + col] = *(const double2*)&sm[row * (RP + 2) + col];
+  }
 }
 
 // A copy the compiler cannot fold away: a prefetch slot is copied out before its next
@@ -2518,8 +2610,19 @@ static int sg(hipStream_t st, int mode, const float* A, int B, int n, int m, con
   return DMH_OK;
 }
 
+// Whether a batch's Gram chunks go over GRAM_WAVES waves each (times beside
+// gram_partials_mw; the order of the fp64 sums is all that differs).
+static bool gram_multi(int B, int rows) {
+  const char* env = getenv("DMH_GRAM_MW");
+  if (env) return env[0] == '1';
+  return B <= 64 || (B <= 96 && rows >= 1024);
+}
+
 static int gram(hipStream_t st, const float* Y, int B, int rows, double* part) {
-  if (gram_stage(rows))
+  if (gram_multi(B, rows))
+    hipLaunchKernelGGL(gram_partials_mw, dim3(GRAM_CHUNKS, B), dim3(64 * GRAM_WAVES), 0, st, Y,
+                       rows, part, (const float*)nullptr, 0, (double*)nullptr);
+  else if (gram_stage(rows))
     hipLaunchKernelGGL(gram_partials<true>, dim3(GRAM_CHUNKS, B), dim3(64), 0, st, Y, rows,
                        (long long)rows * RP, part);
   else
@@ -2533,15 +2636,18 @@ static int gram(hipStream_t st, const float* Y, int B, int rows, double* part) {
 // Q transposed, for the split-bf16 skinny GEMMs.
 // need_q = false (with QT given): Q itself is not read afterwards, only QT -- the last
 // pass writes QT alone
+// first: the first orthonormalisation of a call, whose factorization sets w.degen (w.degen is
+// cleared where there is none)
 static int orth(hipStream_t st, const float* Y, float* Q, float* tmp, int B, int rows, int r,
-                int passes, const RsvdWs& w, float* QT = nullptr, bool need_q = true) {
+                int passes, const RsvdWs& w, bool first, float* QT = nullptr, bool need_q = true) {
   const float* src = Y;
   int rc;
   for (int p = 0; p < passes; ++p) {
     const bool last = p == passes - 1;
     float* dst = last ? Q : (p % 2 == 0 ? tmp : Q);
     if ((rc = gram(st, src, B, rows, w.gram))) return rc;
-    hipLaunchKernelGGL(chol_inv, dim3(B), dim3(CHOL_THREADS), 0, st, w.gram, r, w.M, w.degen);
+    hipLaunchKernelGGL(chol_inv, dim3(B), dim3(CHOL_THREADS), 0, st, w.gram, r, w.M, w.degen,
+                       first && p == 0 ? 1 : 0);
     DMH_CHECK_LAUNCH("chol_inv");
     const RightMult rm{src, rows, (long long)rows * RP, w.M,
                        last && QT && !need_q ? (float*)nullptr : dst, (long long)rows * RP,
@@ -2551,6 +2657,7 @@ static int orth(hipStream_t st, const float* Y, float* Q, float* tmp, int B, int
     src = dst;
   }
   if (passes == 0) {
+    if (first && (rc = zero_ints(st, w.degen, B))) return rc;
     if ((rc = pad_to_rp(st, Y, B, rows, RP, Q))) return rc;
     if (QT) {
       hipLaunchKernelGGL(transpose_rp, dim3(ceil_div(rows, 64), B), dim3(256), 0, st, Y, rows, RP,
@@ -2610,7 +2717,6 @@ static int rsvd_core(hipStream_t st, const float* A, const float* Omega, int B, 
                      int r, int niter, int passes, const GateParams& gp, long long* k_out,
                      float* d, const RsvdWs& w) {
   int rc;
-  if ((rc = zero_ints(st, w.degen, B))) return rc;
   const bool fast = sk_fast(n, m);
   if (fast) {
     // split-bf16 path, 3 terms (fp32-accurate) for every product
@@ -2620,12 +2726,12 @@ static int rsvd_core(hipStream_t st, const float* A, const float* Omega, int B, 
     if ((rc = skr(st, A, B, n, m, w.XT, w.Y, d ? w.asq : nullptr))) return rc;
     // (Q is read only after the last power iteration: the earlier orthonormalisations,
     // and every one of Z, feed the next skinny product through their transposes alone)
-    if ((rc = orth(st, w.Y, w.Q, w.U, B, n, r, passes, w, w.QT, niter == 0))) return rc;
+    if ((rc = orth(st, w.Y, w.Q, w.U, B, n, r, passes, w, true, w.QT, niter == 0))) return rc;
     for (int it = 0; it < niter; ++it) {
       if ((rc = skc(st, A, B, n, m, w.QT, w.Z, w))) return rc;
-      if ((rc = orth(st, w.Z, w.Zq, w.V, B, m, r, passes, w, w.XT, false))) return rc;
+      if ((rc = orth(st, w.Z, w.Zq, w.V, B, m, r, passes, w, false, w.XT, false))) return rc;
       if ((rc = skr(st, A, B, n, m, w.XT, w.Y, nullptr))) return rc;
-      if ((rc = orth(st, w.Y, w.Q, w.U, B, n, r, passes, w, w.QT, it == niter - 1))) return rc;
+      if ((rc = orth(st, w.Y, w.Q, w.U, B, n, r, passes, w, false, w.QT, it == niter - 1))) return rc;
     }
     if ((rc = skc(st, A, B, n, m, w.QT, w.Bt, w))) return rc;
   } else {
@@ -2633,17 +2739,17 @@ static int rsvd_core(hipStream_t st, const float* A, const float* Omega, int B, 
     if ((rc = sg(st, SG_ROWSTREAM, A, B, n, m, Omega, r, r, (long long)m * r, w.Y,
                  (long long)n * RP, d ? w.asq : nullptr)))
       return rc;
-    if ((rc = orth(st, w.Y, w.Q, w.U, B, n, r, passes, w))) return rc;
+    if ((rc = orth(st, w.Y, w.Q, w.U, B, n, r, passes, w, true))) return rc;
     for (int it = 0; it < niter; ++it) {
       // Z = orth(A^T Q) ; Q = orth(A Z)
       if ((rc = sg(st, SG_COLSTREAM, A, B, n, m, w.Q, RP, RP, (long long)n * RP, w.Z,
                    (long long)m * RP)))
         return rc;
-      if ((rc = orth(st, w.Z, w.Zq, w.V, B, m, r, passes, w))) return rc;
+      if ((rc = orth(st, w.Z, w.Zq, w.V, B, m, r, passes, w, false))) return rc;
       if ((rc = sg(st, SG_ROWSTREAM, A, B, n, m, w.Zq, RP, RP, (long long)m * RP, w.Y,
                    (long long)n * RP)))
         return rc;
-      if ((rc = orth(st, w.Y, w.Q, w.U, B, n, r, passes, w))) return rc;
+      if ((rc = orth(st, w.Y, w.Q, w.U, B, n, r, passes, w, false))) return rc;
     }
     // Bp^T = A^T Q (m x RP)
     if ((rc = sg(st, SG_COLSTREAM, A, B, n, m, w.Q, RP, RP, (long long)n * RP, w.Bt,
@@ -2653,7 +2759,10 @@ static int rsvd_core(hipStream_t st, const float* A, const float* Omega, int B, 
   // H = Bp Bp^T = Gram of Bp^T (and Q^T Q for d, in the same launch)
   if (d) {
     const dim3 gg(2 * GRAM_CHUNKS, B);
-    if (gram_stage(m) && gram_stage(n))
+    if (gram_multi(B, n))
+      hipLaunchKernelGGL(gram_partials_mw, gg, dim3(64 * GRAM_WAVES), 0, st, w.Bt, m, w.gram, w.Q,
+                         n, w.gramq);
+    else if (gram_stage(m) && gram_stage(n))
       hipLaunchKernelGGL((gram_partials_pair<true, true>), gg, dim3(64), 0, st, w.Bt, m, w.gram,
                          w.Q, n, w.gramq);
     else if (gram_stage(m))
@@ -2752,9 +2861,8 @@ int dmh_orth(hipStream_t stream, const float* X, int batch, int rows, int r, int
     return DMH_EWORKSPACE;
   }
   // pad X (rows x r) into Y (rows x RP), orthonormalise, copy out r columns
-  int rc = zero_ints(stream, w.degen, batch);
-  if (!rc) rc = pad_to_rp(stream, X, batch, rows, r, w.Y);
-  if (!rc) rc = orth(stream, w.Y, w.Q, w.U, batch, rows, r, passes, w);
+  int rc = pad_to_rp(stream, X, batch, rows, r, w.Y);
+  if (!rc) rc = orth(stream, w.Y, w.Q, w.U, batch, rows, r, passes, w, true);
   if (rc) return rc;
   const int gb = ceil_div((long long)rows * r, 256) > 4096 ? 4096 : ceil_div((long long)rows * r, 256);
   hipLaunchKernelGGL(copy_cols, dim3(gb, batch), dim3(256), 0, stream, w.Q, rows, r, Q);

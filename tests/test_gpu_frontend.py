@@ -405,3 +405,23 @@ def test_clip_sketch_width_edges(N, m, kind):
         assert torch.equal(k.cpu(), ko), scale
         assert torch.allclose(d.cpu(), do, rtol=1e-4), scale
         assert rel(X0.cpu(), X0o) < 1e-4, scale
+
+
+@pytest.mark.parametrize("mw", ["0", "1"])
+@pytest.mark.parametrize("rows,r", [(1, 1), (5, 5), (33, 8), (64, 9), (127, 64), (1001, 33), (3000, 64)])
+def test_orth_row_chunks(N, rows, r, mw, monkeypatch):
+    """CholeskyQR with one and with four waves per row chunk of the Gram, at row counts that
+    leave chunks and waves short or empty, and sketch widths at the edges of the Cholesky's
+    panels: Q against fp64 (Q is X L^-T rounded to fp32, an error of kappa(X) eps; Gaussian X
+    with a unit diagonal added keeps kappa(X) < 100 here) and Q^T Q = I to the same."""
+    monkeypatch.setenv("DMH_GRAM_MW", mw)
+    X = torch.randn(3, rows, r, generator=torch.Generator().manual_seed(rows + r))
+    X[:, torch.arange(r), torch.arange(r)] += 2.0 * r ** 0.5
+    Q = N.orth(X.to(DEV), 1).cpu().double()
+    Xd = X.double()
+    L = torch.linalg.cholesky(Xd.mT @ Xd)
+    want = torch.linalg.solve_triangular(L, Xd.mT, upper=False).mT
+    kappa = float(torch.linalg.cond(Xd).max())
+    assert kappa < 100
+    assert rel(Q, want) < kappa * 2.0 ** -23
+    assert float((Q.mT @ Q - torch.eye(r, dtype=torch.float64)).abs().max()) < kappa * 2.0 ** -22
