@@ -10,8 +10,7 @@
 // Kernels:
 //   skinny_gemm<ROWS>   C = A X       (n x RP)   fp32 MFMA 32x32x2, A streamed by rows
 //   skinny_gemm<COLS>   C = A^T Y     (m x RP)   fp32 MFMA 32x32x2, A streamed by columns
-//                       (both for the shapes sk_fast() leaves out: n or m not a
-//                       multiple of 8, or a matrix of 2 GiB or more)
+//                       (both for the shapes sk_fast() leaves out: a matrix of 2 GiB or more)
 //   sk_rows             C = A X       (n x RP)   split-bf16 MFMA 16x16x32, X staged in LDS
 //   sk_cols, sk_reduce  C = A^T Y     (m x RP)   split-bf16 MFMA 32x32x16, row-split partials
 //   gram_partials       partial fp64 Gram Y^T Y over row chunks (gram_partials_pair: two)
@@ -346,7 +345,8 @@ __global__ __launch_bounds__(CHOL_THREADS) void chol_inv(const double* __restric
 
 // C (rows x RP) = Y (rows x RP) * M (RP x RP), per matrix; 64 rows per workgroup,
 // a 4 x 4 output block per thread.  CT (optional): the same product transposed,
-// RP x ldct per matrix (the layout the skinny GEMMs read their small operand in).
+// RP x ldct per matrix, zero from rows to ldct (the layout the skinny GEMMs read their
+// small operand in).
 struct RightMult {
   const float* Y; int rows; long long y_bs;
   const float* M;
@@ -407,12 +407,13 @@ __device__ __forceinline__ void right_mult_tile(const RightMult& p, int b, int r
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     float* dst = CTb + (long long)(4 * tx + k) * ldct + row0;
-    if (row0 + 3 < rows && (ldct & 3) == 0) {
+    // (rows past the last come out zero: they fill CT's rows up to its pitch)
+    if (row0 + 3 < ldct && (ldct & 3) == 0) {
       *(float4*)dst = make_float4(acc[0][k], acc[1][k], acc[2][k], acc[3][k]);
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (row0 + i < rows) dst[i] = acc[i][k];
+        if (row0 + i < ldct) dst[i] = acc[i][k];
     }
   }
 }
@@ -431,7 +432,8 @@ __global__ __launch_bounds__(256) void right_mult_pair(RightMult p, RightMult q)
 }
 
 // dst (RP x ldd per matrix) = src^T for src (rows x cols, leading dim lds), zero
-// for the columns cols..RP-1: the transposed layout of the skinny GEMMs' small operand.
+// for the columns cols..RP-1 and from rows to ldd (< rows + 64): the transposed layout of the
+// skinny GEMMs' small operand.
 __global__ __launch_bounds__(256) void transpose_rp(const float* __restrict__ src, int rows,
                                                     int cols, int lds, long long s_bs,
                                                     float* __restrict__ dst, int ldd) {
@@ -446,7 +448,7 @@ __global__ __launch_bounds__(256) void transpose_rp(const float* __restrict__ sr
   for (int e = tid; e < 64 * RP; e += 256) {
     const int c = e / 64, rr = e % 64;
     const int row = r0 + rr;
-    if (row < rows) dst[(long long)b * RP * ldd + (long long)c * ldd + row] = t[rr][c];
+    if (row < ldd) dst[(long long)b * RP * ldd + (long long)c * ldd + row] = t[rr][c];
   }
 }
 
@@ -495,6 +497,27 @@ __device__ __forceinline__ f32x16 mfma_split(const bf16x8 (&a)[SPLITS], const bf
   return acc;
 }
 
+// The same six products, the five smaller ones in an accumulator of their own: the sum of the
+// leading products then rounds once per MFMA instead of six times.
+__device__ __forceinline__ void mfma_split_sep(const bf16x8 (&a)[3], const bf16x8 (&b)[3],
+                                               f32x16& acc, f32x16& low) {
+  low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[1], low, 0, 0, 0);
+  low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[2], low, 0, 0, 0);
+  low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b[0], low, 0, 0, 0);
+  low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[1], low, 0, 0, 0);
+  low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[0], low, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], acc, 0, 0, 0);
+}
+__device__ __forceinline__ void mfma_split16_sep(const bf16x8 (&a)[3], const bf16x8 (&b)[3],
+                                                 f32x4& acc, f32x4& low) {
+  low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[1], low, 0, 0, 0);
+  low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[2], low, 0, 0, 0);
+  low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], b[0], low, 0, 0, 0);
+  low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[1], low, 0, 0, 0);
+  low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[0], low, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[0], acc, 0, 0, 0);
+}
+
 constexpr int SKR_ROWS = 256;   // rows of A per sk_rows workgroup (4 waves x 64)
 constexpr int SKC_COLS = 256;   // columns of A per sk_cols workgroup (4 waves x 64)
 // sk_cols workgroups to aim for (row splits).  Fewer splits than a full second round
@@ -502,6 +525,10 @@ constexpr int SKC_COLS = 256;   // columns of A per sk_cols workgroup (4 waves x
 // splits vs 412 at 3; square group (720) 200 us at 1 split vs 217 at 2.
 constexpr int SKC_TARGET = 720;
 constexpr int SK_MAXS = 16;     // maximum row splits of sk_cols
+// Column blocks up to which a split may go down to 128 rows (us of a front-end at 256 / 128
+// rows: 6 x (1001, 333), 12 blocks, 238 / 226; 4 x (768, 768), 12, 281 / 272; (3072, 768), 3,
+// 299 / 296; but 12 x (3072, 768), 36, 414 / 428; 24 x (1024, 1024), 96, 502 / 525).
+constexpr int SKC_FEW = 24;
 
 // The small operand S of a skinny product (RP x lds fp32, row c = its column c) is the
 // first MFMA operand: lane l supplies row 32 cb + l % 32 and 8 contraction indices.  A
@@ -1184,13 +1211,137 @@ __global__ __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(1, 1)))
   }
 }
 
+// sk_rows for batches too small to give every compute unit 256-row workgroups, and for any
+// width m: a workgroup takes 16 NRB rows, its four waves one 16-column block of C each, so the
+// waves share the rows (read through L1) and the staged chunk of X.  Same products in the same
+// order per accumulator as sk_rows: C is bit-identical.  The loads of A are 4-byte aligned
+// 16-byte buffer loads.  RAG (m % 4 != 0): the step that holds the end of the rows loads its
+// floats one by one, so that nothing past a row is read; XT is zero from m to ldxt.  SEP as in
+// sk_cols.  (Whole
+// front-ends on either: beside skr_rows.)
+template <int SPLITS, int NRB, bool RAG, bool SEP>
+__global__ __launch_bounds__(256) void sk_rows_small(const float* __restrict__ A, int n, int m,
+                                                     const float* __restrict__ XT, int ldxt,
+                                                     float* __restrict__ C, double* __restrict__ asq) {
+  __shared__ __attribute__((aligned(16))) bf16 xl[2 * SK_BUF];
+  const int b = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int r0 = blockIdx.x * 16 * NRB;
+  A += (long long)b * n * m;
+  XT += (long long)b * RP * ldxt;
+  C += (long long)b * n * RP;
+  const __amdgpu_buffer_rsrc_t ar = sk_rsrc(A, (long long)n * m);
+  const __amdgpu_buffer_rsrc_t xr = sk_rsrc(XT, (long long)RP * ldxt);
+  unsigned abase[NRB];   // byte offset of the lane's first float, SK_OOB for rows >= n
+#pragma unroll
+  for (int rb = 0; rb < NRB; ++rb) {
+    const int i = r0 + 16 * rb + l16;
+    abase[rb] = i < n ? (unsigned)((long long)i * m + 4 * g) * 4u : SK_OOB;
+  }
+  f32x4 acc[NRB], low[NRB];
+#pragma unroll
+  for (int rb = 0; rb < NRB; ++rb)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[rb][e] = low[rb][e] = 0.f;
+  double sq = 0.0;
+  const bool sumsq = asq && wave == 0;
+  const int nch = (m + SK_KC - 1) / SK_KC;
+  auto load = [&](int ks, float4 (&a)[NRB][2]) {
+    if (RAG && 32 * ks + 32 > m) {   // uniform; steps past the end load zeros here too
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int rb = 0; rb < NRB; ++rb) {
+          float e[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int k = 32 * ks + 16 * h + q;
+            const unsigned off = k + 4 * g < m ? abase[rb] + (unsigned)k * 4u : SK_OOB;
+            e[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ar, (int)off, 0, 0));
+          }
+          a[rb][h] = make_float4(e[0], e[1], e[2], e[3]);
+        }
+      return;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int k = 32 * ks + 16 * h;
+      const bool kin = RAG || k + 4 * g < m;
+#pragma unroll
+      for (int rb = 0; rb < NRB; ++rb)
+        a[rb][h] = sk_ld4(ar, kin ? abase[rb] + (unsigned)k * 4u : SK_OOB);
+    }
+  };
+  SkStage stg;
+  sk_stage_load(stg, xr, ldxt, 0, m, tid);
+  float4 ab[2][NRB][2];
+  load(0, ab[0]);
+  load(1, ab[1]);
+  sk_pin(stg);
+  sk_stage_store<SPLITS, true>(stg, xl, tid);
+  sk_stage_load(stg, xr, ldxt, SK_KC, m, tid);
+  sk_barrier();
+  for (int ch = 0; ch < nch; ++ch) {
+    const bf16* buf = xl + (ch & 1) * SK_BUF;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int ks = 2 * ch + p;
+      float4 ac[NRB][2];
+#pragma unroll
+      for (int rb = 0; rb < NRB; ++rb)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) ac[rb][h] = sk_mov(ab[p][rb][h]);
+      load(ks + 2, ab[p]);
+      bf16x8 xs[SPLITS];
+#pragma unroll
+      for (int s = 0; s < SPLITS; ++s)
+        xs[s] = *(const bf16x8*)(buf + s * SK_TERM + (16 * wave + l16) * SK_PITCH + 32 * p + 8 * g);
+#pragma unroll
+      for (int rb = 0; rb < NRB; ++rb) {
+        const float4 lo = ac[rb][0], hi = ac[rb][1];
+        const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        if (sumsq) {
+          float f = 0.f;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) f = fmaf(v[e], v[e], f);
+          sq += (double)f;
+        }
+        bf16x8 as[SPLITS];
+        split_bf16<SPLITS>(v, as);
+        if constexpr (SEP) mfma_split16_sep(xs, as, acc[rb], low[rb]);
+        else mfma_split16<SPLITS>(xs, as, acc[rb]);
+      }
+    }
+    sk_pin(stg);
+    sk_stage_store<SPLITS, true>(stg, xl + ((ch + 1) & 1) * SK_BUF, tid);
+    sk_barrier();
+    sk_stage_load(stg, xr, ldxt, (ch + 2) * SK_KC, m, tid);
+  }
+#pragma unroll
+  for (int rb = 0; rb < NRB; ++rb) {
+    const int i = r0 + 16 * rb + l16;
+    if (i < n)
+      *(float4*)&C[(long long)i * RP + 16 * wave + 4 * g] =
+          make_float4(acc[rb][0] + low[rb][0], acc[rb][1] + low[rb][1], acc[rb][2] + low[rb][2],
+                      acc[rb][3] + low[rb][3]);
+  }
+  if (sumsq) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
+    if (lane == 0) asq[(long long)b * gridDim.x + blockIdx.x] = sq;
+  }
+}
+
 // Partial C = A^T Y over the rows [s * rps, (s+1) * rps) of split s = blockIdx.y:
 // part[s][b] (m x RP) = sum_i A[i][j] Y[i][c], with Y given transposed: YT (RP x
 // ldyt), YT[c][i] = Y[i][c] (staged in LDS like sk_rows' X).  Wave w owns 64 columns
 // of A; lane l reads the columns j0 + 2 l32 + {0, 1} of 8 consecutive rows, i.e. two
-// 32-column MFMA blocks (block e holds the columns j0 + 2 l32 + e).  Needs m % 2 == 0,
-// n % 8 == 0 and rps % 16 == 0.
-template <int SPLITS>
+// 32-column MFMA blocks (block e holds the columns j0 + 2 l32 + e).  Needs rps % 16 == 0 and
+// YT zero from n to ldyt (a multiple of 8); rows past n load zeros.  ODD (m odd): the lane of
+// the last column alone loads the pair that ends with it.  SEP: mfma_split_sep (the shapes
+// that the fp32 matrix cores had before, whose error it stays below).
+template <int SPLITS, bool ODD = false, bool SEP = false>
 __global__ __launch_bounds__(256) void sk_cols(const float* __restrict__ A, int n, int m,
                                                const float* __restrict__ YT, int ldyt, int rps,
                                                float* __restrict__ part) {
@@ -1205,19 +1356,20 @@ __global__ __launch_bounds__(256) void sk_cols(const float* __restrict__ A, int 
   A += (long long)b * n * m;
   YT += (long long)b * RP * ldyt;
   const int ib = s * rps, ie = min(n, ib + rps);
-  f32x16 acc[2][2];   // [e][cb]
+  f32x16 acc[2][2], low[SEP ? 2 : 1][SEP ? 2 : 1];   // [e][cb]
 #pragma unroll
   for (int e = 0; e < 2; ++e)
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[e][cb][v] = 0.f;
+      for (int v = 0; v < 16; ++v) acc[e][cb][v] = low[SEP ? e : 0][SEP ? cb : 0][v] = 0.f;
   const int nch = (ie - ib + SK_KC - 1) / SK_KC;
   const __amdgpu_buffer_rsrc_t ar = sk_rsrc(A, (long long)n * m);
   const __amdgpu_buffer_rsrc_t yr = sk_rsrc(YT, (long long)RP * ldyt);
   // rows ib + 16 ks + 8 hk .. +7 of the lane's two columns (a step at or past nk, or a
   // column beyond m, loads zeros)
-  const unsigned cbase = jin ? (unsigned)jl * 4u : SK_OOB;
+  const bool edge = ODD && jl == m - 1;   // (jl > 0, as m > 1)
+  const unsigned cbase = jin ? (unsigned)(edge ? jl - 1 : jl) * 4u : SK_OOB;
   auto load = [&](int ks, float2 (&a)[8]) {
     const int i0 = ib + 16 * ks + 8 * hk;
     const bool iin = i0 < ie;            // 8-row groups are whole
@@ -1243,7 +1395,10 @@ __global__ __launch_bounds__(256) void sk_cols(const float* __restrict__ A, int 
       const int ks = ch * (SK_KC / 16) + p;
       float2 ac[8];
 #pragma unroll
-      for (int t = 0; t < 8; ++t) ac[t] = sk_mov(ab[p & 1][t]);
+      for (int t = 0; t < 8; ++t) {
+        ac[t] = sk_mov(ab[p & 1][t]);
+        if (ODD) ac[t].x = edge ? ac[t].y : ac[t].x;
+      }
       load(ks + 2, ab[p & 1]);
       bf16x8 as[2][SPLITS], ys[2][SPLITS];
       {
@@ -1256,7 +1411,10 @@ __global__ __launch_bounds__(256) void sk_cols(const float* __restrict__ A, int 
 #pragma unroll
       for (int e = 0; e < 2; ++e)
 #pragma unroll
-        for (int cb = 0; cb < 2; ++cb) acc[e][cb] = mfma_split<SPLITS>(ys[cb], as[e], acc[e][cb]);
+        for (int cb = 0; cb < 2; ++cb) {
+          if constexpr (SEP) mfma_split_sep(ys[cb], as[e], acc[e][cb], low[e][cb]);
+          else acc[e][cb] = mfma_split<SPLITS>(ys[cb], as[e], acc[e][cb]);
+        }
     }
     // (after the last chunk this stages zeros nobody reads: no branch in the loop)
     sk_pin(stg);
@@ -1264,12 +1422,20 @@ __global__ __launch_bounds__(256) void sk_cols(const float* __restrict__ A, int 
     sk_barrier();
     sk_stage_load(stg, yr, ldyt, ib + (ch + 2) * SK_KC, ie, tid);
   }
+  if constexpr (SEP) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[e][cb][v] += low[e][cb][v];
+  }
   // D[c][col] = C[j][c], col = l32 -> j = j0 + 2 l32 + e
   float* pb = part + ((long long)s * nb + b) * m * RP;
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     const int j = jl + e;
-    if (!jin) continue;
+    if (ODD ? j >= m : !jin) continue;
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
@@ -2506,13 +2672,35 @@ struct RsvdWs {
 
 static size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// The split-bf16 skinny GEMMs need m and n to be multiples of 8; other shapes run the
-// fp32-MFMA kernels.
-// The split-bf16 skinny products: shapes they cover (their buffer-descriptor offsets
-// are 32-bit, below SK_OOB).
-static bool sk_fast(int n, int m) {
-  return n % 8 == 0 && m % 8 == 0 && (long long)n * m * 4 < (1LL << 31) &&
-         (long long)RP * n * 4 < (1LL << 31);
+// The split-bf16 skinny products cover every shape whose operands their buffer descriptors
+// address with 32-bit offsets (below SK_OOB); larger ones run the fp32-MFMA kernels.
+static int sk_pitch(int rows) { return (rows + 7) & ~7; }
+static bool sk_fast(int n, int m) {   // (m = 1: sk_cols reads columns in pairs)
+  return m > 1 && (long long)n * m * 4 < (1LL << 31) && (long long)RP * sk_pitch(n) * 4 < (1LL << 31);
+}
+
+// n or m no multiple of 8: these shapes ran on the fp32 matrix cores (skinny_gemm), and keep
+// the low-order terms of the split products apart (SEP), with an error below theirs: d and X0
+// against 64 bits, 6 x (1001, 333) 1.45e-6 and 1.31e-6 -> 6.0e-7 and 5.2e-7, 4 x (4100, 1025)
+// 4.5e-7 and 9.9e-7 -> 2.3e-7 and 3.2e-7; 13 shapes 0.28 to 0.61 of it.  6 x (1001, 333): 23
+// us per product A X and 61 per A^T Y on skinny_gemm, whole front-end 325 -> 232 us.
+static bool sk_ragged(int n, int m) { return n % 8 != 0 || m % 8 != 0; }
+
+// Rows of A per workgroup of the A X product: SKR_ROWS (sk_rows, sk_rows_dtl), or 16, 32 or 64
+// (sk_rows_small), all with the same products.  us of a front-end at 16 / 32 / 64 / 256 rows:
+// (3072, 768) 299 / 306 / 334 / 336, 4 x (3072, 768) 342 / 338 / 345 / 347, 12 x (768, 768) 322
+// / 318 / 327 / 329, 24 x (1024, 1024) 507 / 483 / 502 / 450, 24 x (1280, 320) 302 / 288 / 284
+// / 267; 24 x (2051, 513), ragged and so only on sk_rows_small, 602 / 563 / 559.
+static int skr_rows(int B, int n, int m) {
+  const char* env = getenv("DMH_SKR_ROWS");
+  const int want = env ? atoi(env) : 0;
+  const bool rag = sk_ragged(n, m);
+  if (getenv("DMH_SKR_DTL") && !rag) return SKR_ROWS;   // (compares the 256-row kernels)
+  if (want == 16 || want == 32 || want == 64 || (want == SKR_ROWS && !rag)) return want;
+  const long long blocks = (long long)B * ceil_div(n, 16);   // 16-row blocks
+  if (blocks <= 512) return 16;
+  if (blocks <= 1024) return 32;
+  return rag ? 64 : SKR_ROWS;
 }
 
 static int zero_ints(hipStream_t st, int* p, int count) {
@@ -2532,12 +2720,13 @@ static int pad_to_rp(hipStream_t st, const float* src, int B, int rows, int cols
   return DMH_OK;
 }
 
-// Row splits of sk_cols: about SKC_TARGET workgroups in all, at least 256 rows each.
+// Row splits of sk_cols: about SKC_TARGET workgroups in all, at least 256 rows each (128 where
+// there are few column blocks).
 static void sk_splits(int B, int n, int m, int* S, int* rps) {
   const long long wgs = (long long)ceil_div(m, SKC_COLS) * (B > 0 ? B : 1);
   int s = (int)((SKC_TARGET + wgs - 1) / wgs);
   s = s < 1 ? 1 : (s > SK_MAXS ? SK_MAXS : s);
-  while (s > 1 && n / s < 256) --s;
+  while (s > 1 && n / s < (wgs <= SKC_FEW ? 128 : 256)) --s;
   int r = ceil_div(n, s);
   r = (r + 15) / 16 * 16;
   *S = ceil_div(n, r);
@@ -2566,7 +2755,7 @@ static RsvdWs rsvd_layout(void* base, int B, int n, int m) {
   w.s = (float*)take((size_t)B * RP * sizeof(float));
   w.gram = (double*)take((size_t)B * GRAM_CHUNKS * RP * RP * sizeof(double));
   w.gramq = (double*)take((size_t)B * GRAM_CHUNKS * RP * RP * sizeof(double));
-  w.asq = (double*)take((size_t)B * ceil_div(n, SG_ROWS) * sizeof(double));
+  w.asq = (double*)take((size_t)B * ceil_div(n, 16) * sizeof(double));
   w.k64 = (long long*)take((size_t)B * sizeof(long long));
   w.kint = (int*)take((size_t)B * sizeof(int));
   w.degen = (int*)take((size_t)B * sizeof(int));
@@ -2575,8 +2764,8 @@ static RsvdWs rsvd_layout(void* base, int B, int n, int m) {
   if (sk_fast(n, m)) {
     int S, rps;
     sk_splits(B, n, m, &S, &rps);
-    w.XT = (float*)take((size_t)B * RP * m * sizeof(float));
-    w.QT = (float*)take((size_t)B * RP * n * sizeof(float));
+    w.XT = (float*)take((size_t)B * RP * sk_pitch(m) * sizeof(float));
+    w.QT = (float*)take((size_t)B * RP * sk_pitch(n) * sizeof(float));
     w.part = (float*)take((size_t)S * B * m * RP * sizeof(float));
   }
   w.bytes = off;
@@ -2635,7 +2824,7 @@ static int gram(hipStream_t st, const float* Y, int B, int rows, double* part) {
 // Q = orth(Y) by CholeskyQR (Y, Q: rows x RP), `passes` times; QT (optional, RP x rows):
 // Q transposed, for the split-bf16 skinny GEMMs.
 // need_q = false (with QT given): Q itself is not read afterwards, only QT -- the last
-// pass writes QT alone
+// pass writes QT alone; QT's pitch is sk_pitch(rows)
 // first: the first orthonormalisation of a call, whose factorization sets w.degen (w.degen is
 // cleared where there is none)
 static int orth(hipStream_t st, const float* Y, float* Q, float* tmp, int B, int rows, int r,
@@ -2651,7 +2840,7 @@ static int orth(hipStream_t st, const float* Y, float* Q, float* tmp, int B, int
     DMH_CHECK_LAUNCH("chol_inv");
     const RightMult rm{src, rows, (long long)rows * RP, w.M,
                        last && QT && !need_q ? (float*)nullptr : dst, (long long)rows * RP,
-                       last ? QT : (float*)nullptr, rows};
+                       last ? QT : (float*)nullptr, sk_pitch(rows)};
     hipLaunchKernelGGL(right_mult, dim3(ceil_div(rows, 64), B), dim3(256), 0, st, rm);
     DMH_CHECK_LAUNCH("right_mult");
     src = dst;
@@ -2661,29 +2850,44 @@ static int orth(hipStream_t st, const float* Y, float* Q, float* tmp, int B, int
     if ((rc = pad_to_rp(st, Y, B, rows, RP, Q))) return rc;
     if (QT) {
       hipLaunchKernelGGL(transpose_rp, dim3(ceil_div(rows, 64), B), dim3(256), 0, st, Y, rows, RP,
-                         RP, (long long)rows * RP, QT, rows);
+                         RP, (long long)rows * RP, QT, sk_pitch(rows));
       DMH_CHECK_LAUNCH("orth transpose");
     }
   }
   return DMH_OK;
 }
 
-// Y (n x RP) = A XT^T with the split-bf16 kernel (XT: RP x m); asq optional
+// Y (n x RP) = A XT^T with the split-bf16 kernel (XT: RP x sk_pitch(m)); asq optional
 static int skr(hipStream_t st, const float* A, int B, int n, int m, const float* XT, float* Y,
                double* asq) {
-  dim3 grid(ceil_div(n, SKR_ROWS), B);
+  const int rows = skr_rows(B, n, m), ld = sk_pitch(m);
+  dim3 grid(ceil_div(n, rows), B);
   // the direct-to-LDS variant needs whole 64-index chunks; DMH_SKR_DTL=0 selects the
   // register-load kernel (same results) for comparisons
   const char* e = getenv("DMH_SKR_DTL");
-  if (m % SK_KC == 0 && !(e && e[0] == '0'))
-    hipLaunchKernelGGL((sk_rows_dtl<3, 8>), grid, dim3(512), 0, st, A, n, m, XT, m, Y, asq);
+#define DMH_SKR_LAUNCH(NRB, RAG, SEP)                                                         \
+  hipLaunchKernelGGL((sk_rows_small<3, NRB, RAG, SEP>), grid, dim3(256), 0, st, A, n, m, XT,  \
+                     ld, Y, asq)
+#define DMH_SKR_SMALL(NRB)                                                                    \
+  do {                                                                                        \
+    if (m % 4) DMH_SKR_LAUNCH(NRB, true, true);                                               \
+    else if (sk_ragged(n, m)) DMH_SKR_LAUNCH(NRB, false, true);                               \
+    else DMH_SKR_LAUNCH(NRB, false, false);                                                   \
+  } while (0)
+  if (rows == 16) DMH_SKR_SMALL(1);
+  else if (rows == 32) DMH_SKR_SMALL(2);
+  else if (rows == 64) DMH_SKR_SMALL(4);
+  else if (m % SK_KC == 0 && !(e && e[0] == '0'))
+    hipLaunchKernelGGL((sk_rows_dtl<3, 8>), grid, dim3(512), 0, st, A, n, m, XT, ld, Y, asq);
   else
-    hipLaunchKernelGGL(sk_rows<3>, grid, dim3(256), 0, st, A, n, m, XT, m, Y, asq);
+    hipLaunchKernelGGL(sk_rows<3>, grid, dim3(256), 0, st, A, n, m, XT, ld, Y, asq);
+#undef DMH_SKR_SMALL
+#undef DMH_SKR_LAUNCH
   DMH_CHECK_LAUNCH("sk_rows");
   return DMH_OK;
 }
 
-// C (m x RP) = A^T YT^T with the split-bf16 kernel (YT: RP x n), row splits reduced
+// C (m x RP) = A^T YT^T with the split-bf16 kernel (YT: RP x sk_pitch(n)), row splits reduced
 // in order
 static int skc(hipStream_t st, const float* A, int B, int n, int m, const float* YT, float* C,
                const RsvdWs& w) {
@@ -2691,7 +2895,15 @@ static int skc(hipStream_t st, const float* A, int B, int n, int m, const float*
   sk_splits(B, n, m, &S, &rps);
   dim3 grid(ceil_div(m, SKC_COLS), S, B);
   // one split: the kernel writes C itself
-  hipLaunchKernelGGL(sk_cols<3>, grid, dim3(256), 0, st, A, n, m, YT, n, rps, S == 1 ? C : w.part);
+  if (m % 2)
+    hipLaunchKernelGGL((sk_cols<3, true, true>), grid, dim3(256), 0, st, A, n, m, YT, sk_pitch(n),
+                       rps, S == 1 ? C : w.part);
+  else if (sk_ragged(n, m))
+    hipLaunchKernelGGL((sk_cols<3, false, true>), grid, dim3(256), 0, st, A, n, m, YT, sk_pitch(n),
+                       rps, S == 1 ? C : w.part);
+  else
+    hipLaunchKernelGGL((sk_cols<3>), grid, dim3(256), 0, st, A, n, m, YT, sk_pitch(n), rps,
+                       S == 1 ? C : w.part);
   DMH_CHECK_LAUNCH("sk_cols");
   if (S == 1) return DMH_OK;
   const long long per = (long long)B * m * RP;
@@ -2721,7 +2933,7 @@ static int rsvd_core(hipStream_t st, const float* A, const float* Omega, int B, 
   if (fast) {
     // split-bf16 path, 3 terms (fp32-accurate) for every product
     hipLaunchKernelGGL(transpose_rp, dim3(ceil_div(m, 64), B), dim3(256), 0, st, Omega, m, r, r,
-                       (long long)m * r, w.XT, m);
+                       (long long)m * r, w.XT, sk_pitch(m));
     DMH_CHECK_LAUNCH("transpose Omega");
     if ((rc = skr(st, A, B, n, m, w.XT, w.Y, d ? w.asq : nullptr))) return rc;
     // (Q is read only after the last power iteration: the earlier orthonormalisations,
@@ -2780,12 +2992,12 @@ static int rsvd_core(hipStream_t st, const float* A, const float* Omega, int B, 
     // the gate ratio, every deflated direction lies within the gate window)
     hipLaunchKernelGGL(eig_head_gate, dim3(B), dim3(EH_THREADS), 0, st, w.gram, gp, w.degen, w.s,
                        RP, w.Ub, w.UbS, k_out, w.kint, w.cw, w.cr, w.gramq, w.asq,
-                       ceil_div(n, fast ? SKR_ROWS : SG_ROWS), d, w.wflag);
+                       ceil_div(n, fast ? skr_rows(B, n, m) : SG_ROWS), d, w.wflag);
     DMH_CHECK_LAUNCH("eig_head_gate");
   } else {
     hipLaunchKernelGGL(eig_gate, dim3(B), dim3(EG_THREADS), 0, st, w.gram, gp, w.degen, w.s, RP,
                        w.Ub, w.UbS, k_out, w.kint, w.cw, w.cr, d ? w.gramq : nullptr,
-                       d ? w.asq : nullptr, ceil_div(n, fast ? SKR_ROWS : SG_ROWS), d,
+                       d ? w.asq : nullptr, ceil_div(n, fast ? skr_rows(B, n, m) : SG_ROWS), d,
                        d ? w.wflag : nullptr);
     DMH_CHECK_LAUNCH("eig_gate");
   }
@@ -2897,8 +3109,15 @@ int dmh_project(hipStream_t stream, const float* Q, const float* A, int batch, i
   int rc = zero_ints(stream, w.degen, batch);
   if (!rc) rc = pad_to_rp(stream, Q, batch, n, r, w.Q);
   if (rc) return rc;
-  rc = sg(stream, SG_COLSTREAM, A, batch, n, m, w.Q, RP, RP, (long long)n * RP, w.Bt,
-              (long long)m * RP);
+  if (sk_fast(n, m)) {
+    hipLaunchKernelGGL(transpose_rp, dim3(ceil_div(n, 64), batch), dim3(256), 0, stream, Q, n, r, r,
+                       (long long)n * r, w.QT, sk_pitch(n));
+    DMH_CHECK_LAUNCH("transpose Q");
+    rc = skc(stream, A, batch, n, m, w.QT, w.Bt, w);
+  } else {
+    rc = sg(stream, SG_COLSTREAM, A, batch, n, m, w.Q, RP, RP, (long long)n * RP, w.Bt,
+            (long long)m * RP);
+  }
   if (rc) return rc;
   if ((rc = gram(stream, w.Bt, batch, m, w.gram))) return rc;
   GateParams gp{r, 1, 0.f, 0.f, 1.f};

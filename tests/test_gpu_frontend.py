@@ -425,3 +425,46 @@ def test_orth_row_chunks(N, rows, r, mw, monkeypatch):
     assert kappa < 100
     assert rel(Q, want) < kappa * 2.0 ** -23
     assert float((Q.mT @ Q - torch.eye(r, dtype=torch.float64)).abs().max()) < kappa * 2.0 ** -22
+
+
+@pytest.mark.parametrize("n,m", [(20, 20), (64, 33), (131, 131), (257, 66), (1001, 333), (515, 130), (900, 90)])
+def test_skinny_products_of_any_width(N, n, m, monkeypatch):
+    """A X and A^T Y at widths that are no multiple of 2, 4 or 8 and row counts that leave the
+    last block and the last 8-row group short: every row-block size gives the same U, s, V and k
+    bit for bit, the divisor (its sums of squares in another order) and X0 agree to fp32
+    rounding, and the result is the oracle's.  A is filled to the end of its allocation's last
+    row with neighbours that a read past a row or past the matrix would pick up."""
+    from defmuon_amd import synthetic as S
+    A = torch.stack([S.spiked_matrix(n, m, seed=5 * b + n, n_spikes=2 if m > 60 else 0, hi=40.0, lo=20.0)
+                     for b in range(3)])
+    r, kw = O.sketch_dims(m)
+    Om = O.draw_omega(3, m, r, 17)
+    hold = torch.full((A.numel() + 64,), float("nan"), device=DEV)
+    Ad = hold[:A.numel()].view(A.shape)
+    Ad.copy_(A)
+    outs = []
+    for rows in ("16", "32", "64"):
+        monkeypatch.setenv("DMH_SKR_ROWS", rows)
+        X0, k, d = N.rmfro_clip(Ad, Om.to(DEV), kw, O.GATE_RATIO, O.DEFLATE_THRESH, O.DIVISOR_PAD)
+        outs.append([t.cpu() for t in (*N.rsvd(Ad, Om.to(DEV)), k, d, X0)])
+    for o in outs[1:]:
+        for a, b in zip(o[:4], outs[0][:4]):
+            assert torch.equal(a, b)
+        assert rel(o[4], outs[0][4]) < 1e-6 and rel(o[5], outs[0][5]) < 1e-6
+    X0o, ko, do = O.rmfro_clip(A, Om, out_dtype=torch.float32)
+    assert torch.equal(outs[0][3], ko)
+    assert torch.allclose(outs[0][4], do, rtol=1e-4)
+    assert rel(outs[0][5], X0o) < 1e-4
+
+
+@pytest.mark.parametrize("n,m,r", [(40, 13, 13), (1001, 333, 18), (300, 300, 64)])
+def test_project_of_any_width(N, n, m, r):
+    """Rayleigh-Ritz on the split products: s and the reconstruction Q Q^T A = U S V^T against
+    fp64 (1e-5: fp32 sums over n, and U and V in fp32)."""
+    g = torch.Generator().manual_seed(n + m)
+    A = torch.randn(2, n, m, generator=g)
+    Q = torch.linalg.qr(torch.randn(2, n, r, generator=g))[0]
+    U, s, V = (t.cpu().double() for t in N.project(Q.to(DEV), A.to(DEV)))
+    B = Q.double().mT @ A.double()
+    assert rel(s, torch.linalg.svdvals(B)) < 1e-5
+    assert rel((U * s[:, None, :]) @ V.mT, Q.double() @ B) < 1e-5
