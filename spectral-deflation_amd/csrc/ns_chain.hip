@@ -1018,7 +1018,16 @@ __global__ __launch_bounds__(C::THREADS) void gemm_ring(GemmArgs g) {
 // ---------------------------------------------------------------------------
 // entry: Frobenius norm partials, then scale + cast + pack into padded T and W
 // ---------------------------------------------------------------------------
-constexpr int NORM_CHUNKS = 64;
+constexpr int NORM_CHUNKS = 256;   // at most; see norm_chunks
+
+// Workgroups (and partial sums) per matrix: about 8 four-element loads per thread.  64 of them
+// whatever the size took 12.3 us for one 768 x 3072 matrix (36 loads per thread) and 9.7 for
+// 3 x (1280, 1280); now 5.3 and 5.9.  From the
+// shape alone, so that a matrix's norm does not depend on its batch.
+__host__ __device__ inline int norm_chunks(int rows, int cols) {
+  const long long c = ((long long)rows * cols + 8191) / 8192;
+  return c < 1 ? 1 : (c > NORM_CHUNKS ? NORM_CHUNKS : (int)c);
+}
 
 struct InView {
   const void* x; int dtype;            // 0 fp32, 1 bf16
@@ -1032,17 +1041,27 @@ __device__ __forceinline__ float load_in(const InView& v, int b, int r, int c) {
   return bf2f(((const bf16*)v.x)[off]);
 }
 
-// Sum of squares of one matrix of the input, NORM_CHUNKS partials per matrix (fp64,
+// the 256 threads' values summed, in every thread (the same order every time)
+__device__ __forceinline__ double block_sum(double v, int tid) {
+  __shared__ double part[4];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  if ((tid & 63) == 0) part[tid >> 6] = v;
+  __syncthreads();
+  return (part[0] + part[1]) + (part[2] + part[3]);
+}
+
+// Sum of squares of one matrix of the input, norm_chunks() partials per matrix (fp64,
 // per element), one workgroup per partial.  When the matrix's rows are contiguous
 // and back to back (column stride 1, row stride = cols) the matrix is one run of
 // rows * cols elements, read in 16-byte loads from its first 16-byte boundary on;
 // otherwise each workgroup takes a range of rows and reads them element by element.
 __global__ __launch_bounds__(256) void entry_norm_partials(InView v, double* partials) {
-  const int b = blockIdx.y, chunk = blockIdx.x, tid = threadIdx.x;
+  const int b = blockIdx.y, chunk = blockIdx.x, tid = threadIdx.x, nch = gridDim.x;
   double s = 0.0;
   if (v.cs == 1 && v.rs == v.cols) {
     const long long total = (long long)v.rows * v.cols;
-    const long long per = (total + NORM_CHUNKS - 1) / NORM_CHUNKS;
+    const long long per = (total + nch - 1) / nch;
     const long long lo = (long long)chunk * per;
     const long long hi = lo + per < total ? lo + per : total;
     const int vec = v.dtype == 0 ? 4 : 8;   // elements per 16 bytes
@@ -1077,7 +1096,7 @@ __global__ __launch_bounds__(256) void entry_norm_partials(InView v, double* par
       s += (double)x * (double)x;
     }
   } else {
-    const int rpc = (v.rows + NORM_CHUNKS - 1) / NORM_CHUNKS;
+    const int rpc = (v.rows + nch - 1) / nch;
     const int r0 = chunk * rpc, r1 = r0 + rpc < v.rows ? r0 + rpc : v.rows;
     for (int r = r0; r < r1; ++r)
       for (int c = tid; c < v.cols; c += 256) {
@@ -1085,14 +1104,8 @@ __global__ __launch_bounds__(256) void entry_norm_partials(InView v, double* par
         s += (double)x * (double)x;
       }
   }
-  __shared__ double red[256];
-  red[tid] = s;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (tid < w) red[tid] += red[tid + w];
-    __syncthreads();
-  }
-  if (tid == 0) partials[b * NORM_CHUNKS + chunk] = red[0];
+  s = block_sum(s, tid);
+  if (tid == 0) partials[b * NORM_CHUNKS + chunk] = s;
 }
 
 // Pack 64x64 tiles of T (i < np rows, j < mp cols) into the chain's block layout.
@@ -1109,15 +1122,11 @@ __global__ __launch_bounds__(256) void entry_pack(InView v, int in_tall, int sca
   const int i0 = blockIdx.y * 64, j0 = blockIdx.x * 64;
   float den = 1.f;
   if (scale_mode) {
-    __shared__ float s_den;
-    if (tid == 0) {
-      double s = 0.0;
-      for (int c = 0; c < NORM_CHUNKS; ++c) s += partials[b * NORM_CHUNKS + c];
-      const float nrm = (float)sqrt(s);
-      s_den = scale_mode == 2 ? nrm * 1.01f + 1e-7f : nrm + 1e-7f;
-    }
-    __syncthreads();
-    den = s_den;
+    // (every thread gets the same sum)
+    const double s = block_sum(tid < norm_chunks(v.rows, v.cols) ? partials[b * NORM_CHUNKS + tid] : 0.0,
+                               tid);
+    const float nrm = (float)sqrt(s);
+    den = scale_mode == 2 ? nrm * 1.01f + 1e-7f : nrm + 1e-7f;
   }
   bf16* Tb = T + (long long)b * np * mp;
   const float* xf = (const float*)v.x;
@@ -1509,7 +1518,7 @@ int dmh_ns_chain(hipStream_t stream, const void* x, int x_dtype, int batch, int 
   }
   InView v{x, x_dtype, x_bstride, x_rstride, x_cstride, rows, cols};
   if (entry_mode) {
-    hipLaunchKernelGGL(entry_norm_partials, dim3(NORM_CHUNKS, batch), dim3(256), 0, stream, v,
+    hipLaunchKernelGGL(entry_norm_partials, dim3(norm_chunks(rows, cols), batch), dim3(256), 0, stream, v,
                        w.partials);
     DMH_CHECK_LAUNCH("entry_norm_partials");
   }
