@@ -1222,14 +1222,17 @@ ChainWs chain_ws(void* ws, int batch, const ChainDims& d) {
   ChainWs w{};
   const size_t tw = (size_t)batch * d.np * d.mp;
   const size_t sq = (size_t)batch * d.mp * d.mp;
-  const size_t part = (size_t)batch * NORM_CHUNKS * sizeof(double);
-  w.bytes = (2 * tw + 2 * sq) * sizeof(bf16) + ((part + 255) / 256) * 256;
+  const size_t tail = (size_t)batch * 64 * sizeof(double);
+  w.bytes = (2 * tw + 2 * sq) * sizeof(bf16) + ((tail + 255) / 256) * 256;
   if (!ws) return w;
   w.T0 = (bf16*)ws;
   w.T1 = w.T0 + tw;
   w.A = w.T1 + tw;
   w.B = w.A + sq;
-  w.partials = (double*)(w.B + sq);
+  // the norm's partial sums end the workspace: its tail and the last bytes of B, which nothing
+  // writes before K2 (at least 128 KB per matrix, of which they take 1.5)
+  static_assert((NORM_CHUNKS - 64) * sizeof(double) <= 256 * 256 * sizeof(bf16), "fits B");
+  w.partials = (double*)((char*)ws + w.bytes) - (size_t)batch * NORM_CHUNKS;
   return w;
 }
 
