@@ -2,9 +2,11 @@
 
 The reference's plain Muon step calls the factorizer once per parameter
 (muon.py:361-386): at GPT-2 sizes that is a stream of small, occupancy-bound
-launches.  `install()` switches Muon to one library launch per (matrix shape,
-dtype, orientation), the way deflation_cutoff.install() (deflation_cutoff.py:46-112)
-changes Muon's behaviour from outside; every parameter's update is unchanged
+launches.  Muon's own step takes buckets of parameters (Muon.PLAIN_BUCKET elements)
+with one library launch per (matrix shape, dtype, orientation) of a bucket;
+`install()` lifts the limit, the way deflation_cutoff.install()
+(deflation_cutoff.py:46-112) changes Muon's behaviour from outside.  Every
+parameter's update is that of its own factorizer call
 (Muon._muon_step_plain_grouped).  The deflated arms batch by shape already.
 """
 
@@ -12,7 +14,7 @@ _INSTALLED = [False]
 
 
 def install():
-    """Enable the grouped plain-arm step for every Muon instance (idempotent)."""
+    """One bucket per parameter group for every Muon instance (idempotent)."""
     if _INSTALLED[0]:
         return
     _INSTALLED[0] = True
@@ -21,7 +23,7 @@ def install():
 
 
 def uninstall():
-    """Back to one factorizer call per parameter (the reference's loop)."""
+    """Back to buckets of Muon.PLAIN_BUCKET elements."""
     from defmuon_amd.optim.muon import Muon
     Muon.GROUPED_PLAIN = False
     _INSTALLED[0] = False

@@ -37,13 +37,19 @@ def zeropower_via_newtonschulz5(G, steps):
     return out.reshape(G.shape)
 
 
+# the built-in factorizers, whatever the module's names are bound to later
+_NS5, _PE = zeropower_via_newtonschulz5, PolarExpress
+
+
 def plain_group_chains(stacks, talls, entry_mode, sched):
     """The plain arm's chain (ns_chain with entry normalisation) over each stacked
     group, [polar factors] in group order.  With several groups on a GPU every group
     runs on a side stream of its own, the largest first: a small group's launches
     leave most compute units idle, which the other groups' launches fill.  Each result
-    equals that of ns_chain on its group alone."""
-    if len(stacks) < 2 or not stacks[0].is_cuda:
+    equals that of ns_chain on its group alone.  Under capture all stay on the captured
+    stream."""
+    if (len(stacks) < 2 or not stacks[0].is_cuda
+            or torch.cuda.is_current_stream_capturing()):
         return [_native.ns_chain(X, t, entry_mode, sched) for X, t in zip(stacks, talls)]
     from defmuon_amd.optim.deflation_batched import _side_streams
     dev = stacks[0].device
@@ -315,57 +321,98 @@ class Muon(torch.optim.Optimizer):
             out.append(d)
         return out
 
-    # -- the plain arms, grouped by matrix shape (grouped_plain.install()) -------
-    GROUPED_PLAIN = False
+    # -- the plain arms, grouped by matrix shape ---------------------------------
+    GROUPED_PLAIN = False   # grouped_plain.install(): buckets of any size
+
+    # Elements of the parameters that share a plain-arm step's launches.  A chain alone on
+    # one GPT-2-small matrix leaves most compute units idle (about 170 us each, sixteen in a
+    # row for four layers: a step 2980 us one by one, 1036 in a bucket; one layer of width 64
+    # is bound by its launches, 754 at one factorizer call each, 540 here).  2^26 elements are
+    # nine GPT-2-small layers or three of GPT-2 large, several times what fills the GPU, and
+    # bound the stacks, polar factors and workspaces of a step to about 1.2 GB beside the
+    # largest parameter's own.
+    PLAIN_BUCKET = 1 << 26
+
+    def _plain_buckets(self, params):
+        """`params` (those with gradients) in runs of at most PLAIN_BUCKET elements on one
+        device, in their order."""
+        buckets, size = [], 0
+        for p in params:
+            if p.grad is None:
+                continue
+            if (not buckets or p.device != buckets[-1][0].device
+                    or (size + p.numel() > self.PLAIN_BUCKET and not self.GROUPED_PLAIN)):
+                buckets.append([])
+                size = 0
+            buckets[-1].append(p)
+            size += p.numel()
+        return buckets
 
     def _muon_step_plain_grouped(self, group, params, lr, weight_decay, momentum):
         """The plain-arm update (muon.py:361-386) with one library launch per
-        (matrix shape, dtype, orientation) instead of one factorizer call per
-        parameter.  The orientation is the one the factorizer itself would pick
-        for the parameter (size(0) > size(1) for ns5, muon.py:30; size(-2) >
+        (matrix shape, dtype, orientation) of a bucket of parameters instead of one
+        factorizer call per parameter.  The orientation is the one the factorizer itself
+        would pick for the parameter (size(0) > size(1) for ns5, muon.py:30; size(-2) >
         size(-1) for PolarExpress, polar_express.py:25), the entry normalisation
         is per matrix, and the matrices of a launch do not interact, so every
         update equals the per-parameter one.  Returns False (nothing done) for a
         factorizer other than the built-in two."""
         fac = self.polar_factorizer
         steps = group["ns_steps"]
-        if fac is zeropower_via_newtonschulz5:
+        if fac is _NS5:
             mode, sched = 1, [NS_ABC] * steps
-        elif fac is PolarExpress:
+        elif fac is _PE:
             mode, sched = 2, pe_schedule(steps)
         else:
             return False
+        for bucket in self._plain_buckets(params):
+            self._plain_bucket_step(group, bucket, lr, weight_decay, momentum, mode, sched)
+        return True
+
+    def _plain_bucket_step(self, group, params, lr, weight_decay, momentum, mode, sched):
+        # (the fused update asks for the learning rate without gradient and update)
+        fused = (type(self).adjust_lr_for_muon is Muon.adjust_lr_for_muon
+                 and self._fused_glue_ok(group, params))
         groups = {}
         for p in params:
             g = p.grad
-            if g is None:
-                continue
             state = self.state[p]
             if "momentum_buffer" not in state:
                 state["momentum_buffer"] = torch.zeros_like(g)
-            buf = state["momentum_buffer"]
-            buf.mul_(momentum).add_(g)
-            g = g.add(buf, alpha=momentum) if group["nesterov"] else buf
+            if not fused:
+                buf = state["momentum_buffer"]
+                buf.mul_(momentum).add_(g)
+                g = g.add(buf, alpha=momentum) if group["nesterov"] else buf
             gq = self._qkv_split(p, g)
             tall = gq.size(0) > gq.size(1) if mode == 1 else gq.size(-2) > gq.size(-1)
             X = as_batch(gq)
-            groups.setdefault((tuple(X.shape[1:]), X.dtype, tall), []).append((p, g, X))
-        keys = list(groups)
-        stacks = [groups[k][0][2] if len(groups[k]) == 1 else torch.cat([X for _, _, X in groups[k]])
-                  for k in keys]
-        outs = plain_group_chains(stacks, [k[2] for k in keys], mode, sched)
-        for key, out in zip(keys, outs):
-            es = groups[key]
+            e = {"p": p, "g": g, "X": X, "tr": False, "nb": X.shape[0]}
+            groups.setdefault((tuple(X.shape[1:]), X.dtype, tall), []).append(e)
+        stacks = []
+        for (shape, _, _), es in groups.items():
+            if fused:   # momentum and stack in one launch; X is not read
+                X = torch.empty((sum(e["nb"] for e in es),) + shape, dtype=torch.float32,
+                                device=params[0].device)
+                _native.momentum_stack(self._glue_params(es, shape), momentum,
+                                       group["nesterov"], X)
+            else:
+                X = es[0]["X"] if len(es) == 1 else torch.cat([e["X"] for e in es])
+            stacks.append(X)
+        outs = plain_group_chains(stacks, [k[2] for k in groups], mode, sched)
+        for ((shape, _, _), es), out in zip(groups.items(), outs):
+            if fused:
+                _native.apply_update(self._glue_params(es, shape, lr, weight_decay, group), out)
+                continue
             off = 0
-            for p, g, X in es:
-                u = out[off:off + X.shape[0]].reshape(g.shape)
-                off += X.shape[0]
+            for e in es:
+                p, g = e["p"], e["g"]
+                u = out[off:off + e["nb"]].reshape(g.shape)
+                off += e["nb"]
                 adjusted_lr = self.adjust_lr_for_muon(lr, group["rms_scaling"],
                                                       group["nuclear_scaling"], p.shape,
                                                       g.bfloat16(), u)
                 p.data.mul_(1 - lr * weight_decay)
                 p.data.add_(u, alpha=-adjusted_lr)
-        return True
 
     # -- the AdamW backup as one library launch per group (FUSED_GLUE) ----------
     ADAMW_TABLES_KEPT = 4   # device tables kept per parameter group
@@ -431,9 +478,7 @@ class Muon(torch.optim.Optimizer):
             if self.batched_deflation and params:
                 self._muon_step_batched(group, params, lr, weight_decay, momentum)
                 params = []
-            if (self.GROUPED_PLAIN and params
-                    and self._muon_step_plain_grouped(group, params, lr, weight_decay,
-                                                      momentum)):
+            if params and self._muon_step_plain_grouped(group, params, lr, weight_decay, momentum):
                 params = []
             for p in params:
                 g = p.grad

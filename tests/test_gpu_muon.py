@@ -248,6 +248,44 @@ def test_grouped_plain_step_equals_per_parameter_loop(muon_mod, arm):
         assert torch.equal(results[False][k], results[True][k]), k
 
 
+@pytest.mark.parametrize("arm", ["ns5", "polarexpress"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("bucket", [None, 3 * D * D, 0])
+def test_plain_buckets_equal_factorizer_calls(muon_mod, arm, dtype, bucket):
+    """Buckets of any size move every parameter and momentum bit for bit like one
+    factorizer call per parameter (a wrapped factorizer keeps that loop), W_QKV, ragged and
+    strided parameters among them; a parameter without a gradient stays."""
+    muon, DB = muon_mod
+    results = {}
+    for loop in (True, False):
+        params = _named_params(11)
+        g = torch.Generator().manual_seed(12)
+        params["ragged.weight"] = torch.nn.Parameter(torch.randn(77, 131, generator=g).to(DEV))
+        params["idle.weight"] = torch.nn.Parameter(torch.randn(64, 32, generator=g).to(DEV))
+        if dtype != torch.float32:
+            params = {k: torch.nn.Parameter(p.detach().to(dtype)) for k, p in params.items()}
+            params["strided.weight"] = torch.nn.Parameter(
+                torch.randn(96, 200, generator=g).to(DEV).T)
+        opt = muon.Muon(list(params.items()), lr=0.01, weight_decay=0.1, polar_method=arm,
+                        nesterov=bucket is None)
+        if loop:
+            fac = opt.polar_factorizer
+            opt.polar_factorizer = lambda G, steps: fac(G, steps)
+        elif bucket is not None:
+            opt.PLAIN_BUCKET = bucket
+        for _ in range(2):
+            for k, p in params.items():
+                if k != "idle.weight":
+                    p.grad = torch.randn(p.shape, generator=g).to(DEV, p.dtype)
+            opt.step()
+        results[loop] = [p.detach() for p in params.values()] + [
+            opt.state[p]["momentum_buffer"] for p in params.values()
+            if "momentum_buffer" in opt.state[p]]
+    assert len(results[True]) == len(results[False])
+    for x, y in zip(results[True], results[False]):
+        assert torch.equal(x, y)
+
+
 @pytest.mark.parametrize("nesterov", [True, False])
 def test_fused_glue_equals_torch_ops(muon_mod, nesterov):
     """dmh_momentum_stack / dmh_apply_update (one launch per shape group) leave
