@@ -191,8 +191,14 @@ class Muon(torch.optim.Optimizer):
     FUSED_GLUE = True
 
     def _fused_glue_ok(self, group, params):
-        """The fused glue covers rms scaling on contiguous fp32 GPU tensors."""
+        """The fused glue covers rms scaling on contiguous fp32 GPU tensors, with the
+        learning rate and the block split of this class: a subclass's, an instance's or a
+        patched one has the gradient and the update to look at, which only the torch ops
+        hand over."""
         if not self.FUSED_GLUE or group["nuclear_scaling"]:
+            return False
+        if any(getattr(getattr(self, name), "__func__", None) is not fn
+               for name, fn in _BUILT_IN.items()):
             return False
         for p in params:
             g = p.grad
@@ -370,9 +376,7 @@ class Muon(torch.optim.Optimizer):
         return True
 
     def _plain_bucket_step(self, group, params, lr, weight_decay, momentum, mode, sched):
-        # (the fused update asks for the learning rate without gradient and update)
-        fused = (type(self).adjust_lr_for_muon is Muon.adjust_lr_for_muon
-                 and self._fused_glue_ok(group, params))
+        fused = self._fused_glue_ok(group, params)
         groups = {}
         for p in params:
             g = p.grad
@@ -525,3 +529,7 @@ class Muon(torch.optim.Optimizer):
                 p.data.mul_(1 - lr * weight_decay)
                 p.data.add_(g, alpha=-lr / scale)
         return loss
+
+
+# what the fused glue computes by itself, whatever the class's names are bound to later
+_BUILT_IN = {"adjust_lr_for_muon": Muon.adjust_lr_for_muon, "_qkv_split": Muon._qkv_split}

@@ -286,6 +286,47 @@ def test_plain_buckets_equal_factorizer_calls(muon_mod, arm, dtype, bucket):
         assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("arm", ["ns5", "deflated_ns_cut"])
+@pytest.mark.parametrize("how", ["subclass", "class", "instance", "split"])
+def test_own_learning_rate_or_split_gets_gradient_and_update(muon_mod, monkeypatch, arm, how):
+    """A learning rate or block split of the user's own, put in by any route, is called as the
+    torch ops call it (gradient and update in hand): parameters bit for bit as with the fused
+    glue off."""
+    muon, DB = muon_mod
+    from defmuon_amd.optim import deflation_cutoff
+    deflation_cutoff.install()
+    built_in = muon.Muon.adjust_lr_for_muon
+
+    def lr_by_gradient(self, lr, rms, nuc, shape, grad, update):
+        assert grad.shape == update.shape == tuple(shape)
+        return built_in(self, lr, rms, nuc, shape, grad, update) * float(grad.abs().mean())
+
+    def halves(self, p, g):
+        return g.reshape(2, g.shape[0] // 2, g.shape[1])
+
+    results = {}
+    for fused in (False, True):
+        params = _named_params(21)
+        grads = _grads(params, 22)
+        cls = muon.Muon
+        if how == "subclass":
+            cls = type("OwnRate", (muon.Muon,), {"adjust_lr_for_muon": lr_by_gradient})
+        elif how == "class":
+            monkeypatch.setattr(muon.Muon, "adjust_lr_for_muon", lr_by_gradient)
+        elif how == "split":
+            cls = type("OwnSplit", (muon.Muon,), {"_qkv_split": halves})
+        opt = cls(list(params.items()), lr=0.01, weight_decay=0.1, polar_method=arm)
+        if how == "instance":
+            opt.adjust_lr_for_muon = lr_by_gradient.__get__(opt)
+        opt.FUSED_GLUE = fused
+        for k, p in params.items():
+            p.grad = grads[k]
+        opt.step()
+        results[fused] = [p.detach() for p in params.values()]
+    for x, y in zip(results[False], results[True]):
+        assert torch.equal(x, y)
+
+
 @pytest.mark.parametrize("nesterov", [True, False])
 def test_fused_glue_equals_torch_ops(muon_mod, nesterov):
     """dmh_momentum_stack / dmh_apply_update (one launch per shape group) leave
