@@ -191,10 +191,10 @@ class Muon(torch.optim.Optimizer):
     FUSED_GLUE = True
 
     def _fused_glue_ok(self, group, params):
-        """The fused glue covers rms scaling on contiguous fp32 GPU tensors, with the
-        learning rate and the block split of this class: a subclass's, an instance's or a
-        patched one has the gradient and the update to look at, which only the torch ops
-        hand over."""
+        """The fused glue covers rms scaling on contiguous fp32 GPU tensors of the
+        parameter's shape and device (it indexes all three flat), with the learning rate
+        and the block split of this class: a subclass's, an instance's or a patched one has
+        the gradient and the update to look at, which only the torch ops hand over."""
         if not self.FUSED_GLUE or group["nuclear_scaling"]:
             return False
         if any(getattr(getattr(self, name), "__func__", None) is not fn
@@ -207,7 +207,7 @@ class Muon(torch.optim.Optimizer):
             buf = self.state[p].get("momentum_buffer")
             ts = (p.data, g) if buf is None else (p.data, g, buf)
             if any(not t.is_cuda or t.dtype != torch.float32 or not t.is_contiguous()
-                   for t in ts) or p.ndim != 2:
+                   or t.shape != p.shape or t.device != p.device for t in ts) or p.ndim != 2:
                 return False
         return True
 

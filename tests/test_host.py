@@ -104,3 +104,36 @@ def test_adjust_lr():
     assert opt.adjust_lr_for_muon(0.1, False, False, (8, 2), None, None) == 0.1
     g = torch.eye(3)
     assert opt.adjust_lr_for_muon(1.0, False, True, (3, 3), g, 2 * g) == pytest.approx(6.0)
+
+
+class _Fake:
+    """What _fused_glue_ok looks at of a tensor: a GPU tensor without a GPU."""
+
+    def __init__(self, shape, device="cuda:0", dtype=torch.float32, contiguous=True):
+        self.shape, self.ndim, self.dtype = torch.Size(shape), len(shape), dtype
+        self.device, self.is_cuda = torch.device(device), device.startswith("cuda")
+        self.is_contiguous = lambda: contiguous
+        self.data, self.grad = self, None
+
+
+@pytest.mark.parametrize("which", ["grad", "momentum_buffer"])
+@pytest.mark.parametrize("bad", [dict(shape=(6, 3)), dict(shape=(3,)), dict(shape=(4, 6)),
+                                 dict(shape=(6, 4), device="cuda:1"), dict(shape=(6, 4), device="cpu"),
+                                 dict(shape=(6, 4), dtype=torch.bfloat16),
+                                 dict(shape=(6, 4), contiguous=False)])
+def test_fused_glue_takes_tensors_of_the_parameters_shape_alone(which, bad):
+    """The fused glue reads and writes rows * cols elements of the gradient and the momentum
+    buffer: a buffer of another shape (a state dict of another model) or device goes to the
+    torch ops, which refuse it."""
+    from defmuon_amd.optim import muon
+    opt = muon.Muon([("w", torch.nn.Parameter(torch.zeros(8, 2)))], polar_method="ns5")
+    p = _Fake((6, 4))
+    p.grad = _Fake((6, 4))
+    group = {"nuclear_scaling": False}
+    opt.state[p]["momentum_buffer"] = _Fake((6, 4))
+    assert opt._fused_glue_ok(group, [p])
+    if which == "grad":
+        p.grad = _Fake(**bad)
+    else:
+        opt.state[p]["momentum_buffer"] = _Fake(**bad)
+    assert not opt._fused_glue_ok(group, [p])
