@@ -14,6 +14,7 @@ the groups' clips run concurrently on separate streams before their chains
 of the others in the batch and of the order the groups run in.
 """
 
+import bisect
 import math
 import os
 
@@ -67,6 +68,14 @@ def plain_group_chains(stacks, talls, entry_mode, sched):
     for s in side:
         main.wait_stream(s)
     return outs
+
+
+def _byte_range(p):
+    """[first, end) of the memory p's elements lie in."""
+    lo = p.data_ptr()
+    if p.numel() == 0:
+        return lo, lo
+    return lo, lo + (1 + sum((n - 1) * st for n, st in zip(p.shape, p.stride()))) * p.element_size()
 
 
 _EXCLUDED = ("embeddings", "embed_tokens", "wte", "lm_head", "wpe")
@@ -341,17 +350,25 @@ class Muon(torch.optim.Optimizer):
 
     def _plain_buckets(self, params):
         """`params` (those with gradients) in runs of at most PLAIN_BUCKET elements on one
-        device, in their order."""
+        device, in their order.  Parameters that share memory (one given twice, tied
+        weights) come in buckets of their own: a bucket reads and writes all of its
+        parameters at once, where the loop takes one after the other."""
         buckets, size = [], 0
         for p in params:
             if p.grad is None:
                 continue
-            if (not buckets or p.device != buckets[-1][0].device
+            lo, hi = _byte_range(p)
+            if buckets:
+                i = bisect.bisect(los, lo)
+                shares = (i > 0 and his[i - 1] > lo) or (i < len(los) and los[i] < hi)
+            if (not buckets or p.device != buckets[-1][0].device or shares
                     or (size + p.numel() > self.PLAIN_BUCKET and not self.GROUPED_PLAIN)):
                 buckets.append([])
-                size = 0
+                size, los, his, i = 0, [], [], 0
             buckets[-1].append(p)
             size += p.numel()
+            los.insert(i, lo)     # the ranges of a bucket, disjoint and in order
+            his.insert(i, hi)
         return buckets
 
     def _muon_step_plain_grouped(self, group, params, lr, weight_decay, momentum):

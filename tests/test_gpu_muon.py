@@ -286,6 +286,32 @@ def test_plain_buckets_equal_factorizer_calls(muon_mod, arm, dtype, bucket):
         assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("nesterov", [True, False])
+def test_plain_buckets_with_shared_memory_equal_factorizer_calls(muon_mod, nesterov):
+    """Tied weights and a parameter given twice are updated one after the other, as by one
+    factorizer call per parameter."""
+    muon, DB = muon_mod
+    results = {}
+    for loop in (True, False):
+        g = torch.Generator().manual_seed(31)
+        a = torch.nn.Parameter(torch.randn(96, 64, generator=g).to(DEV))
+        tied = torch.nn.Parameter(a.data)
+        part = torch.nn.Parameter(a.data[32:64])
+        with pytest.warns(UserWarning, match="duplicate"):
+            opt = muon.Muon([("a", a), ("tied", tied), ("part", part), ("again", a)], lr=0.01,
+                            weight_decay=0.1, nesterov=nesterov)
+        if loop:
+            fac = opt.polar_factorizer
+            opt.polar_factorizer = lambda G, steps: fac(G, steps)
+        for _ in range(2):
+            for p in (a, tied, part):
+                p.grad = torch.randn(p.shape, generator=g).to(DEV)
+            opt.step()
+        results[loop] = [a.detach()] + [opt.state[p]["momentum_buffer"] for p in (a, tied, part)]
+    for x, y in zip(results[True], results[False]):
+        assert torch.equal(x, y)
+
+
 @pytest.mark.parametrize("arm", ["ns5", "deflated_ns_cut"])
 @pytest.mark.parametrize("how", ["subclass", "class", "instance", "split"])
 def test_own_learning_rate_or_split_gets_gradient_and_update(muon_mod, monkeypatch, arm, how):

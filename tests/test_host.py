@@ -137,3 +137,31 @@ def test_fused_glue_takes_tensors_of_the_parameters_shape_alone(which, bad):
     else:
         opt.state[p]["momentum_buffer"] = _Fake(**bad)
     assert not opt._fused_glue_ok(group, [p])
+
+
+def test_plain_buckets_keep_shared_memory_apart():
+    """Parameters that share memory never share a bucket (its launches update all of them at
+    once); neighbours in one buffer do."""
+    from defmuon_amd.optim import muon
+    flat = torch.zeros(40, 8)
+    P = torch.nn.Parameter
+    a, b, c = P(flat[:8]), P(flat[8:24]), P(flat[24:])
+    tied, inner, row = P(flat[8:24]), P(flat[10:12]), P(flat[23:25])
+    flipped = P(flat[:8].T)
+    empty = P(torch.zeros(0, 8))
+    opt = muon.Muon([("w", P(torch.zeros(8, 2)))], polar_method="ns5")
+
+    def buckets(*params):
+        for p in params:
+            p.grad = torch.zeros_like(p)
+        return [[id(p) for p in b] for b in opt._plain_buckets(params)]
+
+    def ids(*groups):
+        return [[id(p) for p in g] for g in groups]
+
+    assert buckets(c, a, b, empty, empty) == ids((c, a, b, empty, empty))
+    assert buckets(a, b, a, c) == ids((a, b), (a, c))
+    assert buckets(a, b, tied, c) == ids((a, b), (tied, c))
+    assert buckets(a, inner, b, c) == ids((a, inner), (b, c))
+    assert buckets(a, b, c, row) == ids((a, b, c), (row,))
+    assert buckets(b, c, flipped, a) == ids((b, c, flipped), (a,))
