@@ -9,6 +9,7 @@ nothing here synchronises.
 """
 
 import ctypes
+import functools
 import os
 
 import torch
@@ -118,6 +119,16 @@ def _workspace(nbytes, device):
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
 
 
+@functools.lru_cache(maxsize=1024)
+def ns_workspace_bytes(batch, rows, cols, orient_tall):
+    """Workspace of ns_chain on a (batch, rows, cols) stack (both sides of a matrix count
+    in multiples of 256)."""
+    nbytes = c_sz()
+    _check(load().dmh_ns_workspace_size(batch, rows, cols, int(bool(orient_tall)),
+                                        ctypes.byref(nbytes)), "dmh_ns_workspace_size")
+    return nbytes.value
+
+
 def ns_chain(X, orient_tall, entry_mode, coeffs, out=None):
     """Run the bf16 polynomial chain on a (batch, rows, cols) stack.
 
@@ -142,14 +153,12 @@ def ns_chain(X, orient_tall, entry_mode, coeffs, out=None):
         return out
     steps = len(coeffs)
     flat = (ctypes.c_double * max(3 * steps, 1))(*[float(v) for t in coeffs for v in t])
-    nbytes = c_sz()
-    _check(lib.dmh_ns_workspace_size(B, R, C, int(bool(orient_tall)), ctypes.byref(nbytes)),
-           "dmh_ns_workspace_size")
-    ws = _workspace(nbytes.value, X.device)
+    nbytes = ns_workspace_bytes(B, R, C, bool(orient_tall))
+    ws = _workspace(nbytes, X.device)
     bs, rs, cs = X.stride()
     rc = lib.dmh_ns_chain(_stream(X.device), c_vp(X.data_ptr()), 0 if X.dtype == torch.float32 else 1,
                           B, R, C, bs, rs, cs, c_vp(out.data_ptr()), int(bool(orient_tall)),
-                          int(entry_mode), flat, steps, c_vp(ws.data_ptr()), nbytes.value)
+                          int(entry_mode), flat, steps, c_vp(ws.data_ptr()), nbytes)
     _check(rc, "dmh_ns_chain")
     return out
 

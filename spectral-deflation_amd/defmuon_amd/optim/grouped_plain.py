@@ -2,7 +2,7 @@
 
 The reference's plain Muon step calls the factorizer once per parameter
 (muon.py:361-386): at GPT-2 sizes that is a stream of small, occupancy-bound
-launches.  Muon's own step takes buckets of parameters (Muon.PLAIN_BUCKET elements)
+launches.  Muon's own step takes buckets of parameters (Muon.PLAIN_BUCKET bytes)
 with one library launch per (matrix shape, dtype, orientation) of a bucket;
 `install()` lifts the limit, the way deflation_cutoff.install()
 (deflation_cutoff.py:46-112) changes Muon's behaviour from outside.  Every
@@ -23,7 +23,7 @@ def install():
 
 
 def uninstall():
-    """Back to buckets of Muon.PLAIN_BUCKET elements."""
+    """Back to buckets of Muon.PLAIN_BUCKET bytes."""
     from defmuon_amd.optim.muon import Muon
     Muon.GROUPED_PLAIN = False
     _INSTALLED[0] = False

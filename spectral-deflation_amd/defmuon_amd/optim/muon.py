@@ -56,17 +56,21 @@ def plain_group_chains(stacks, talls, entry_mode, sched):
     dev = stacks[0].device
     main = torch.cuda.current_stream(dev)
     order = sorted(range(len(stacks)), key=lambda i: -stacks[i].numel())
-    outs = [None] * len(stacks)
+    # Stacks and outputs belong to the current stream, which waits for the side streams before
+    # it goes on, and are held until then: their memory is free for what follows as soon as they
+    # are dropped.  (Shared with record_stream, it would be free once the GPU had got there, and
+    # a host that runs ahead would allocate every bucket of a step anew.)
+    outs = [torch.empty(X.shape, dtype=torch.bfloat16, device=dev) for X in stacks]
     side = _side_streams(dev, len(stacks))
     for s in side:
         s.wait_stream(main)
-    for s, i in zip(side, order):
-        with torch.cuda.stream(s):
-            outs[i] = _native.ns_chain(stacks[i], talls[i], entry_mode, sched)
-        stacks[i].record_stream(s)
-        outs[i].record_stream(main)
-    for s in side:
-        main.wait_stream(s)
+    try:
+        for s, i in zip(side, order):
+            with torch.cuda.stream(s):
+                _native.ns_chain(stacks[i], talls[i], entry_mode, sched, out=outs[i])
+    finally:
+        for s in side:
+            main.wait_stream(s)
     return outs
 
 
@@ -339,17 +343,33 @@ class Muon(torch.optim.Optimizer):
     # -- the plain arms, grouped by matrix shape ---------------------------------
     GROUPED_PLAIN = False   # grouped_plain.install(): buckets of any size
 
-    # Elements of the parameters that share a plain-arm step's launches.  A chain alone on
-    # one GPT-2-small matrix leaves most compute units idle (about 170 us each, sixteen in a
-    # row for four layers: a step 2980 us one by one, 1036 in a bucket; one layer of width 64
-    # is bound by its launches, 754 at one factorizer call each, 540 here).  2^26 elements are
-    # nine GPT-2-small layers or three of GPT-2 large, several times what fills the GPU, and
-    # bound the stacks, polar factors and workspaces of a step to about 1.2 GB beside the
-    # largest parameter's own.
-    PLAIN_BUCKET = 1 << 26
+    # Bytes that the parameters sharing a plain-arm step's launches take beside their gradients
+    # and state (_plain_bytes).  A chain alone on one GPT-2-small matrix leaves most compute
+    # units idle (about 170 us each, sixteen in a row for four layers: a step 2980 us one by one,
+    # 1036 in a bucket; one layer of width 64 is bound by its launches, 754 at one factorizer
+    # call each, 540 here).  1 GiB is nine GPT-2-small layers or three of GPT-2 large, several
+    # times what fills the GPU; a parameter that takes more has a bucket to itself.
+    PLAIN_BUCKET = 1 << 30
 
-    def _plain_buckets(self, params):
-        """`params` (those with gradients) in runs of at most PLAIN_BUCKET elements on one
+    def _plain_view(self, p, t, mode):
+        """The matrices the factorizer takes t (p's gradient, or p itself) for, as a batch, and
+        their orientation (size(0) > size(1) for ns5, muon.py:30; size(-2) > size(-1) for
+        PolarExpress, polar_express.py:25)."""
+        q = self._qkv_split(p, t)
+        tall = q.size(0) > q.size(1) if mode == 1 else q.size(-2) > q.size(-1)
+        return as_batch(q), tall
+
+    def _plain_bytes(self, p, mode):
+        """At most what p adds to its bucket: momentum, stack and polar factor, and the chain's
+        workspace, which pads the matrices (a 4096 x 8 one takes 4.3 MB)."""
+        if p.numel() == 0:
+            return 0
+        X, tall = self._plain_view(p, p.grad, mode)
+        return (p.numel() * (2 * max(p.element_size(), 4) + 2)
+                + _native.ns_workspace_bytes(*X.shape, tall))
+
+    def _plain_buckets(self, params, mode):
+        """`params` (those with gradients) in runs of at most PLAIN_BUCKET bytes on one
         device, in their order.  Parameters that share memory (one given twice, tied
         weights) come in buckets of their own: a bucket reads and writes all of its
         parameters at once, where the loop takes one after the other."""
@@ -358,15 +378,16 @@ class Muon(torch.optim.Optimizer):
             if p.grad is None:
                 continue
             lo, hi = _byte_range(p)
+            need = self._plain_bytes(p, mode)
             if buckets:
                 i = bisect.bisect(los, lo)
                 shares = (i > 0 and his[i - 1] > lo) or (i < len(los) and los[i] < hi)
             if (not buckets or p.device != buckets[-1][0].device or shares
-                    or (size + p.numel() > self.PLAIN_BUCKET and not self.GROUPED_PLAIN)):
+                    or (size + need > self.PLAIN_BUCKET and not self.GROUPED_PLAIN)):
                 buckets.append([])
                 size, los, his, i = 0, [], [], 0
             buckets[-1].append(p)
-            size += p.numel()
+            size += need
             los.insert(i, lo)     # the ranges of a bucket, disjoint and in order
             his.insert(i, hi)
         return buckets
@@ -375,11 +396,10 @@ class Muon(torch.optim.Optimizer):
         """The plain-arm update (muon.py:361-386) with one library launch per
         (matrix shape, dtype, orientation) of a bucket of parameters instead of one
         factorizer call per parameter.  The orientation is the one the factorizer itself
-        would pick for the parameter (size(0) > size(1) for ns5, muon.py:30; size(-2) >
-        size(-1) for PolarExpress, polar_express.py:25), the entry normalisation
-        is per matrix, and the matrices of a launch do not interact, so every
-        update equals the per-parameter one.  Returns False (nothing done) for a
-        factorizer other than the built-in two."""
+        would pick for the parameter (_plain_view), the entry normalisation is per matrix,
+        and the matrices of a launch do not interact, so every update equals the
+        per-parameter one.  Returns False (nothing done) for a factorizer other than the
+        built-in two."""
         fac = self.polar_factorizer
         steps = group["ns_steps"]
         if fac is _NS5:
@@ -388,7 +408,7 @@ class Muon(torch.optim.Optimizer):
             mode, sched = 2, pe_schedule(steps)
         else:
             return False
-        for bucket in self._plain_buckets(params):
+        for bucket in self._plain_buckets(params, mode):
             self._plain_bucket_step(group, bucket, lr, weight_decay, momentum, mode, sched)
         return True
 
@@ -404,9 +424,7 @@ class Muon(torch.optim.Optimizer):
                 buf = state["momentum_buffer"]
                 buf.mul_(momentum).add_(g)
                 g = g.add(buf, alpha=momentum) if group["nesterov"] else buf
-            gq = self._qkv_split(p, g)
-            tall = gq.size(0) > gq.size(1) if mode == 1 else gq.size(-2) > gq.size(-1)
-            X = as_batch(gq)
+            X, tall = self._plain_view(p, g, mode)
             e = {"p": p, "g": g, "X": X, "tr": False, "nb": X.shape[0]}
             groups.setdefault((tuple(X.shape[1:]), X.dtype, tall), []).append(e)
         stacks = []

@@ -250,7 +250,7 @@ def test_grouped_plain_step_equals_per_parameter_loop(muon_mod, arm):
 
 @pytest.mark.parametrize("arm", ["ns5", "polarexpress"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("bucket", [None, 3 * D * D, 0])
+@pytest.mark.parametrize("bucket", [None, 2 << 20, 0])   # all, about three, one parameter
 def test_plain_buckets_equal_factorizer_calls(muon_mod, arm, dtype, bucket):
     """Buckets of any size move every parameter and momentum bit for bit like one
     factorizer call per parameter (a wrapped factorizer keeps that loop), W_QKV, ragged and
@@ -284,6 +284,36 @@ def test_plain_buckets_equal_factorizer_calls(muon_mod, arm, dtype, bucket):
     assert len(results[True]) == len(results[False])
     for x, y in zip(results[True], results[False]):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("shape", [(1024, 8), (8, 2048), (64, 64), (512, 256)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_plain_step_memory_is_one_bucket(muon_mod, shape, dtype):
+    """A step of many buckets, enqueued while the GPU is still busy with earlier work, takes
+    no more memory than one bucket (and the allocator's rounding to 512 bytes) beside
+    parameters, gradients and state."""
+    muon, DB = muon_mod
+    params = [torch.nn.Parameter(torch.randn(*shape, device=DEV).to(dtype)) for _ in range(60)]
+    extra = [torch.nn.Parameter(torch.randn(96, 40, device=DEV).to(dtype)) for _ in range(60)]
+    both = [p for pair in zip(params, extra) for p in pair]    # two groups in every bucket
+    opt = muon.Muon([(f"{i}.weight", p) for i, p in enumerate(both)], lr=0.01)
+    opt.PLAIN_BUCKET = 16 << 20
+    for p in both:
+        p.grad = torch.randn_like(p)
+    assert len(opt._plain_buckets(both, 1)) > 3
+    opt.step()
+    X = torch.randn(4096, 4096, device=DEV)
+    Y = torch.empty_like(X)
+    torch.mm(X, X, out=Y)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    for _ in range(200):       # about 0.2 s of work ahead of the step
+        torch.mm(X, X, out=Y)
+    opt.step()
+    peak = torch.cuda.max_memory_allocated() - before
+    torch.cuda.synchronize()
+    assert peak <= opt.PLAIN_BUCKET + (1 << 17), peak
 
 
 @pytest.mark.parametrize("nesterov", [True, False])

@@ -154,7 +154,7 @@ def test_plain_buckets_keep_shared_memory_apart():
     def buckets(*params):
         for p in params:
             p.grad = torch.zeros_like(p)
-        return [[id(p) for p in b] for b in opt._plain_buckets(params)]
+        return [[id(p) for p in b] for b in opt._plain_buckets(params, 1)]
 
     def ids(*groups):
         return [[id(p) for p in g] for g in groups]
@@ -165,3 +165,36 @@ def test_plain_buckets_keep_shared_memory_apart():
     assert buckets(a, inner, b, c) == ids((a, inner), (b, c))
     assert buckets(a, b, c, row) == ids((a, b, c), (row,))
     assert buckets(b, c, flipped, a) == ids((b, c, flipped), (a,))
+
+
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("shape", [(4096, 8), (16, 4096), (64, 64), (768, 3072), (3 * 256, 256)])
+def test_plain_buckets_count_padded_bytes(shape, mode):
+    """A bucket's stack, polar factors and chain workspaces, as they are allocated, stay within
+    PLAIN_BUCKET (a parameter above it is alone), and a bucket is not broken while the next
+    parameter still fits; no limit under grouped_plain."""
+    from defmuon_amd import _native
+    from defmuon_amd.optim import muon
+    name = "attn.c_attn.weight" if shape[0] == 3 * shape[1] else "mlp.weight"
+    params = [torch.nn.Parameter(torch.zeros(shape)) for _ in range(10)]
+    opt = muon.Muon([(f"{i}.{name}", p) for i, p in enumerate(params)],
+                    polar_method="ns5" if mode == 1 else "polarexpress")
+    for p in params:
+        p.grad = torch.zeros_like(p)
+    nb = 3 if "c_attn" in name else 1
+    rows, cols = shape[0] // nb, shape[1]
+    tall = rows > cols if nb == 1 or mode == 2 else 3 > rows
+
+    def allocated(n):    # fp32 momentum and stack, bf16 polar factors, one workspace
+        return (n * params[0].numel() * (4 + 4 + 2)
+                + _native.ns_workspace_bytes(n * nb, rows, cols, tall))
+
+    for limit in (0, allocated(1), allocated(3) + 100000, allocated(10) + 100000):
+        opt.PLAIN_BUCKET = limit
+        bs = opt._plain_buckets(params, mode)
+        assert [id(p) for b in bs for p in b] == [id(p) for p in params]
+        for b in bs:
+            assert len(b) == 1 or allocated(len(b)) <= limit
+        assert all(allocated(len(b) + 1) > limit - 10 * 4096 for b in bs[:-1])
+    opt.GROUPED_PLAIN, opt.PLAIN_BUCKET = True, 0
+    assert len(opt._plain_buckets(params, mode)) == 1
