@@ -9,8 +9,6 @@ With DEFMUON_DEFL_CUTOFF=N set, the optimizer hard-switches to the plain arm
 
 import os
 
-import torch
-
 from defmuon_amd.optim.deflation_batched import DeflatedNSPolar, DeflatedPEPolar
 
 _env = os.environ.get("DEFMUON_DEFL_CUTOFF")
@@ -44,21 +42,10 @@ def install():
     orig_init = Muon._initialize_polar_factorizer
 
     def warm_post(muon, post):
-        """Run the post-cutoff factorizer once per shape at construction (zeros:
-        the global RNG stays untouched)."""
-        fn = post_fns[post]
-        steps = muon.defaults["ns_steps"]
-        seen = set()
-        for group in muon.param_groups:
-            for p in group["params"]:
-                if not muon.state[p].get("use_muon"):
-                    continue
-                shape = tuple(muon._qkv_split(p, p).shape)
-                key = (shape, p.dtype, p.device)
-                if key not in seen:
-                    seen.add(key)
-                    fn(torch.zeros(shape, dtype=p.dtype, device=p.device), steps)
-        print(f"[deflation_cutoff] warmed {post} for {len(seen)} shapes")
+        """Run the post-cutoff factorizer at construction as the plain step will call it
+        (zeros: the global RNG stays untouched)."""
+        seen = muon._warm_plain(post_fns[post], muon.defaults["ns_steps"])
+        print(f"[deflation_cutoff] warmed {post} for {seen} shapes")
 
     def init_with_cutoff(self, polar_method, polar_args):
         arm = ARMS.get(polar_method)

@@ -135,9 +135,9 @@ class Muon(torch.optim.Optimizer):
         return g
 
     def _warm_polar_compile(self):
-        """Construction-time warm-up (muon.py:167-240): load the library and run
-        each kernel family once on every shape the step will feed it, so first-call
-        costs land before the clock starts.  Zeros for the iteration, randn from a
+        """Construction-time warm-up (muon.py:167-240): load the library and run the
+        polar kernels once on the batches the step will feed them (every parameter with a
+        gradient), so first-call costs land before the clock starts.  Zeros for the iteration, randn from a
         dedicated generator for the clip; the global RNG is never touched."""
         fac = self.polar_factorizer
         steps = self.defaults["ns_steps"]
@@ -165,20 +165,39 @@ class Muon(torch.optim.Optimizer):
                     print(f"warm_polar: warmed the deflated clip and iteration for "
                           f"{len(groups)} tall-shape groups at construction")
             else:
-                seen = set()
-                for group in self.param_groups:
-                    for p in group["params"]:
-                        if not self.state[p].get("use_muon"):
-                            continue
-                        shape = tuple(self._qkv_split(p, p).shape)
-                        key = (shape, p.dtype, p.device)
-                        if key not in seen:
-                            seen.add(key)
-                            fac(torch.zeros(shape, dtype=p.dtype, device=p.device), steps)
+                seen = self._warm_plain(fac, steps)
                 if seen:
-                    print(f"warm_polar: warmed the polar factorizer for {len(seen)} shapes")
+                    print(f"warm_polar: warmed the polar factorizer for {seen} shapes")
         except Exception as e:   # a failed warm-up only moves first-call cost into step 1
             print(f"warm_polar: warm-up failed ({e}); step 1 pays the first-call cost")
+
+    def _warm_plain(self, fac, steps):
+        """Zeros through a plain arm's polar kernels as the step calls them: the built-in two
+        on its buckets' stacks, another factorizer once per shape.  Returns the shapes' count."""
+        seen = set()
+        for group in self.param_groups:
+            params = [p for p in group["params"] if self.state[p].get("use_muon")]
+            plan = self._plain_plan(fac, steps)
+            if plan is not None:
+                mode, sched = plan
+                for bucket in self._plain_buckets(params, mode):
+                    stacks = {}
+                    for p in bucket:
+                        X, tall = self._plain_view(p, p, mode)
+                        key = (tuple(X.shape[1:]), X.dtype, tall)
+                        stacks[key] = stacks.get(key, 0) + X.shape[0]
+                    plain_group_chains(
+                        [torch.zeros((nb,) + shape, dtype=dtype, device=bucket[0].device)
+                         for (shape, dtype, _), nb in stacks.items()],
+                        [tall for _, _, tall in stacks], mode, sched)
+            for p in params:
+                shape = tuple(self._qkv_split(p, p).shape)
+                key = (shape, p.dtype, p.device)
+                if key not in seen:
+                    seen.add(key)
+                    if plan is None:
+                        fac(torch.zeros(shape, dtype=p.dtype, device=p.device), steps)
+        return len(seen)
 
     def _initialize_polar_factorizer(self, polar_method, polar_args):
         if polar_method == "ns5":
@@ -351,8 +370,17 @@ class Muon(torch.optim.Optimizer):
     # times what fills the GPU; a parameter that takes more has a bucket to itself.
     PLAIN_BUCKET = 1 << 30
 
+    @staticmethod
+    def _plain_plan(fac, steps):
+        """(entry mode, schedule) of a built-in plain factorizer, or None."""
+        if fac is _NS5:
+            return 1, [NS_ABC] * steps
+        if fac is _PE:
+            return 2, pe_schedule(steps)
+        return None
+
     def _plain_view(self, p, t, mode):
-        """The matrices the factorizer takes t (p's gradient, or p itself) for, as a batch, and
+        """The matrices the factorizer takes t (p's momentum, or p itself) for, as a batch, and
         their orientation (size(0) > size(1) for ns5, muon.py:30; size(-2) > size(-1) for
         PolarExpress, polar_express.py:25)."""
         q = self._qkv_split(p, t)
@@ -364,19 +392,17 @@ class Muon(torch.optim.Optimizer):
         workspace, which pads the matrices (a 4096 x 8 one takes 4.3 MB)."""
         if p.numel() == 0:
             return 0
-        X, tall = self._plain_view(p, p.grad, mode)
+        X, tall = self._plain_view(p, p, mode)
         return (p.numel() * (2 * max(p.element_size(), 4) + 2)
                 + _native.ns_workspace_bytes(*X.shape, tall))
 
     def _plain_buckets(self, params, mode):
-        """`params` (those with gradients) in runs of at most PLAIN_BUCKET bytes on one
+        """`params` in runs of at most PLAIN_BUCKET bytes on one
         device, in their order.  Parameters that share memory (one given twice, tied
         weights) come in buckets of their own: a bucket reads and writes all of its
         parameters at once, where the loop takes one after the other."""
         buckets, size = [], 0
         for p in params:
-            if p.grad is None:
-                continue
             lo, hi = _byte_range(p)
             need = self._plain_bytes(p, mode)
             if buckets:
@@ -400,15 +426,12 @@ class Muon(torch.optim.Optimizer):
         and the matrices of a launch do not interact, so every update equals the
         per-parameter one.  Returns False (nothing done) for a factorizer other than the
         built-in two."""
-        fac = self.polar_factorizer
-        steps = group["ns_steps"]
-        if fac is _NS5:
-            mode, sched = 1, [NS_ABC] * steps
-        elif fac is _PE:
-            mode, sched = 2, pe_schedule(steps)
-        else:
+        plan = self._plain_plan(self.polar_factorizer, group["ns_steps"])
+        if plan is None:
             return False
-        for bucket in self._plain_buckets(params, mode):
+        mode, sched = plan
+        live = [p for p in params if p.grad is not None]
+        for bucket in self._plain_buckets(live, mode):
             self._plain_bucket_step(group, bucket, lr, weight_decay, momentum, mode, sched)
         return True
 

@@ -198,3 +198,35 @@ def test_plain_buckets_count_padded_bytes(shape, mode):
         assert all(allocated(len(b) + 1) > limit - 10 * 4096 for b in bs[:-1])
     opt.GROUPED_PLAIN, opt.PLAIN_BUCKET = True, 0
     assert len(opt._plain_buckets(params, mode)) == 1
+
+
+@pytest.mark.parametrize("arm", ["ns5", "polarexpress", "deflated_ns_cut"])
+def test_warm_up_runs_the_batches_of_the_step(monkeypatch, arm):
+    """The polar kernels are chosen by their batch: the construction-time warm-up of the plain
+    arms (and of the arm behind a deflation cutoff) runs the stacks that the step will run."""
+    from defmuon_amd.optim import deflation_cutoff as C
+    from defmuon_amd.optim import muon
+    calls = []
+
+    def chains(stacks, talls, mode, sched):
+        calls.append(([(tuple(X.shape), X.dtype) for X in stacks], list(talls), mode, list(sched)))
+        return [torch.zeros(X.shape, dtype=torch.bfloat16) for X in stacks]
+
+    monkeypatch.setattr(muon, "plain_group_chains", chains)
+    C.install()
+    if arm.startswith("deflated"):
+        monkeypatch.setattr(C, "CUTOFF_STEPS", 0)
+    P = torch.nn.Parameter
+    params = [("wte.weight", P(torch.zeros(16, 8)))]
+    for i in range(3):
+        params += [(f"{i}.attn.c_attn.weight", P(torch.zeros(24, 8))),
+                   (f"{i}.mlp.c_fc.weight", P(torch.zeros(32, 8))),
+                   (f"{i}.mlp.c_proj.weight", P(torch.zeros(8, 32, dtype=torch.bfloat16)))]
+    monkeypatch.setattr(muon.Muon, "PLAIN_BUCKET", 5 << 20)
+    opt = muon.Muon(params, polar_method=arm)
+    warm = list(calls)
+    calls.clear()
+    for _, p in params:
+        p.grad = torch.randn_like(p)
+    opt.step()
+    assert len(calls) > 1 and warm == calls
