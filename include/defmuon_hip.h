@@ -58,6 +58,15 @@ int dmh_ns_chain(dmh_stream_t stream, const void* x, int x_dtype, int batch, int
                  int orient_tall, int entry_mode, const double* coeffs, int steps, void* ws,
                  size_t ws_bytes);
 
+/* dmh_ns_chain for a chain that other chains run beside, on other streams of the same GPU:
+ * `beside` is the sum of batch * ceil(rows / 64) * ceil(cols / 64) over those (0: none).  It
+ * decides which kernels run, never the result. */
+int dmh_ns_chain_beside(dmh_stream_t stream, const void* x, int x_dtype, int batch, int rows,
+                        int cols, long long x_bstride, long long x_rstride,
+                        long long x_cstride, void* out, int orient_tall, int entry_mode,
+                        const double* coeffs, int steps, void* ws, size_t ws_bytes,
+                        long long beside);
+
 /* Allocation-free variant of dmh_ns_chain.  It has no counterpart in the reference:
  * it is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same arguments

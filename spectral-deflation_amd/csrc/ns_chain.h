@@ -44,12 +44,14 @@ int chain_check(const char* what, const ChainDims& d);
 ChainWs chain_ws(void* ws, int batch, const ChainDims& d);   // ws == nullptr: sizes only
 
 // The rows and columns of T0 (from the first; multiples of 64) that an entry has to write
-// for chain_run_packed on this batch, its zero padding included.
-void chain_extent(const ChainDims& d, int batch, int* rows, int* cols);
+// for chain_run_packed on this batch, its zero padding included.  beside: as there.
+void chain_extent(const ChainDims& d, int batch, int* rows, int* cols, long long beside = 0);
 
 // Run `steps` iterations from T0 already packed in the workspace; the result
-// goes to `out` (batch, rows, cols) bf16 in the orientation given.
+// goes to `out` (batch, rows, cols) bf16 in the orientation given.  beside: 64 x 64 blocks
+// of the iterates of chains that run at the same time on other streams (chain_cfg).
 int chain_run_packed(hipStream_t stream, const ChainWs& w, int batch, const ChainDims& d,
-                     int orient_tall, const double* coeffs, int steps, bf16* out);
+                     int orient_tall, const double* coeffs, int steps, bf16* out,
+                     long long beside = 0);
 
 }  // namespace dmh

@@ -1354,13 +1354,22 @@ static void phase_tiles(const ChainDims& d, int tile[3]) {
 // multiple of 256 costs gemm_nt_bf16 the padding: from 1.75 times the rings' products on
 // (m = 320, 520, 576; 96 x (576, 576) 1242 -> 932 us) they keep the larger batches too;
 // at 1.5 to 1.74 (m = 448, 833, 1100) it is as fast or faster.
-static void chain_cfg(const ChainDims& d, int batch, int cfg[3]) {
+// The rings are for a GPU that the chain leaves partly idle.  Where other chains run on other
+// streams (`beside`: the 64 x 64 blocks of their iterates), a small group's rings take from a
+// GPU that is full, and the persistent kernel is ahead from 15000 blocks in all on.  us of a
+// plain arm's three groups (4 L square, L tall, L wide) by these rules alone / all persistent:
+// m = 768, L = 4 (6912 blocks) 746 / 805, L = 6 (10368) 971 / 981, L = 9 (15552) 1360 / 1340,
+// L = 12 (20736) 1774 / 1731; m = 1024, L = 4 (12288) 1252 / 1372, L = 6 (18432) 1881 / 1829,
+// L = 8 (24576) 2437 / 2328; m = 640, L = 12 (14400) 1428 / 1517; m = 1280, L = 3 (14400) 1716
+// / 1731, L = 4 (19200) 2242 / 2165, L = 8 (38400) 4324 / 4097.
+static void chain_cfg(const ChainDims& d, int batch, long long beside, int cfg[3]) {
   const long long tn = ceil_div(d.n, CHAIN_BLK), tm = ceil_div(d.m, CHAIN_BLK);
   const long long ts = batch * (tm * (tm + 1) / 2), tt = batch * tn * tm;
   const bool wide = d.mp > 768;
   cfg[0] = ts <= 500 ? RING_64 : ts <= 1000 ? RING_128_DEEP : wide && ts <= 1700 ? RING_128 : RING_NONE;
   cfg[1] = ts <= 1000 ? RING_64 : wide && ts <= 1700 ? RING_128_DEEP : RING_NONE;
   cfg[2] = tt <= 448 ? RING_64 : tt <= 1400 ? RING_128x64 : tt <= 2000 ? RING_128 : RING_NONE;
+  if (beside > 0 && tt + beside >= 15000) cfg[0] = cfg[1] = cfg[2] = RING_NONE;
   // 64 x 64 x 64 products per matrix of either kernel
   int tl[3];
   phase_tiles(d, tl);
@@ -1386,16 +1395,17 @@ static void chain_cfg(const ChainDims& d, int batch, int cfg[3]) {
 // with every phase on gemm_ring nothing past the last 64 x 64 block is read
 static bool all_ring(const int cfg[3]) { return cfg[0] && cfg[1] && cfg[2]; }
 
-void chain_extent(const ChainDims& d, int batch, int* rows, int* cols) {
+void chain_extent(const ChainDims& d, int batch, int* rows, int* cols, long long beside) {
   int cfg[3];
-  chain_cfg(d, batch, cfg);
+  chain_cfg(d, batch, beside, cfg);
   const bool ring = all_ring(cfg);
   *rows = ring ? ceil_div(d.n, CHAIN_BLK) * CHAIN_BLK : d.np;
   *cols = ring ? ceil_div(d.m, CHAIN_BLK) * CHAIN_BLK : d.mp;
 }
 
 int chain_run_packed(hipStream_t stream, const ChainWs& w, int batch, const ChainDims& d,
-                     int orient_tall, const double* coeffs, int steps, bf16* outp) {
+                     int orient_tall, const double* coeffs, int steps, bf16* outp,
+                     long long beside) {
   if (steps == 0) {
     const long long total = (long long)d.n * d.m;
     const int blocks = (int)std::min<long long>((total + 255) / 256, 4096);
@@ -1407,8 +1417,8 @@ int chain_run_packed(hipStream_t stream, const ChainWs& w, int batch, const Chai
   int tl[3];
   phase_tiles(d, tl);
   int cfg[3], nc, mc;
-  chain_cfg(d, batch, cfg);
-  chain_extent(d, batch, &nc, &mc);
+  chain_cfg(d, batch, beside, cfg);
+  chain_extent(d, batch, &nc, &mc, beside);
   // Consecutive launches walk the batch in opposite directions, so each one starts
   // on the matrices the previous one wrote last, which are still in the memory-side
   // cache (the group's operands are several times its size).  The entry pack wrote
@@ -1500,10 +1510,10 @@ int dmh_ns_workspace_size(int batch, int rows, int cols, int orient_tall, size_t
   return DMH_OK;
 }
 
-int dmh_ns_chain(hipStream_t stream, const void* x, int x_dtype, int batch, int rows, int cols,
-                 long long x_bstride, long long x_rstride, long long x_cstride, void* out,
-                 int orient_tall, int entry_mode, const double* coeffs, int steps, void* ws,
-                 size_t ws_bytes) {
+int dmh_ns_chain_beside(hipStream_t stream, const void* x, int x_dtype, int batch, int rows,
+                        int cols, long long x_bstride, long long x_rstride, long long x_cstride,
+                        void* out, int orient_tall, int entry_mode, const double* coeffs,
+                        int steps, void* ws, size_t ws_bytes, long long beside) {
   if (batch == 0) return DMH_OK;
   if (!x || !out || batch < 0 || rows <= 0 || cols <= 0 || steps < 0 ||
       (steps > 0 && !coeffs) || (x_dtype != 0 && x_dtype != 1) || entry_mode < 0 ||
@@ -1526,11 +1536,20 @@ int dmh_ns_chain(hipStream_t stream, const void* x, int x_dtype, int batch, int 
     DMH_CHECK_LAUNCH("entry_norm_partials");
   }
   int er, ec;
-  chain_extent(d, batch, &er, &ec);
+  chain_extent(d, batch, &er, &ec, beside);
   hipLaunchKernelGGL(entry_pack, dim3(ec / 64, er / 64, batch), dim3(256), 0, stream, v,
                      orient_tall, entry_mode, w.partials, d.n, d.m, d.np, d.mp, w.T0);
   DMH_CHECK_LAUNCH("entry_pack");
-  return chain_run_packed(stream, w, batch, d, orient_tall, coeffs, steps, (bf16*)out);
+  return chain_run_packed(stream, w, batch, d, orient_tall, coeffs, steps, (bf16*)out, beside);
+}
+
+int dmh_ns_chain(hipStream_t stream, const void* x, int x_dtype, int batch, int rows, int cols,
+                 long long x_bstride, long long x_rstride, long long x_cstride, void* out,
+                 int orient_tall, int entry_mode, const double* coeffs, int steps, void* ws,
+                 size_t ws_bytes) {
+  return dmh_ns_chain_beside(stream, x, x_dtype, batch, rows, cols, x_bstride, x_rstride,
+                             x_cstride, out, orient_tall, entry_mode, coeffs, steps, ws, ws_bytes,
+                             0);
 }
 
 }  // extern "C"

@@ -28,6 +28,9 @@ _SIGS = {
     "dmh_ns_workspace_size": (c_int, [c_int, c_int, c_int, c_int, ctypes.POINTER(c_sz)]),
     "dmh_ns_chain": (c_int, [c_vp, c_vp, c_int, c_int, c_int, c_int, c_ll, c_ll, c_ll, c_vp,
                              c_int, c_int, ctypes.POINTER(ctypes.c_double), c_int, c_vp, c_sz]),
+    "dmh_ns_chain_beside": (c_int, [c_vp, c_vp, c_int, c_int, c_int, c_int, c_ll, c_ll, c_ll,
+                                    c_vp, c_int, c_int, ctypes.POINTER(ctypes.c_double), c_int,
+                                    c_vp, c_sz, c_ll]),
     "dmh_ns_chain_noalloc": (c_int, [c_vp, c_vp, c_int, c_int, c_int, c_int, c_ll, c_ll, c_ll,
                                      c_vp, c_int, c_int, ctypes.POINTER(ctypes.c_double),
                                      c_int]),
@@ -129,7 +132,12 @@ def ns_workspace_bytes(batch, rows, cols, orient_tall):
     return nbytes.value
 
 
-def ns_chain(X, orient_tall, entry_mode, coeffs, out=None):
+def chain_blocks(X):
+    """64 x 64 blocks of a (batch, rows, cols) stack: what ns_chain's `beside` counts."""
+    return X.shape[0] * -(-X.shape[1] // 64) * -(-X.shape[2] // 64)
+
+
+def ns_chain(X, orient_tall, entry_mode, coeffs, out=None, beside=0):
     """Run the bf16 polynomial chain on a (batch, rows, cols) stack.
 
     orient_tall: the input is the tall operand T of the tall convention
@@ -138,6 +146,8 @@ def ns_chain(X, orient_tall, entry_mode, coeffs, out=None):
     entry_mode: 0 none (input already normalised), 1 divide by ||X||_F + 1e-7,
         2 divide by 1.01 ||X||_F + 1e-7 (norm over the un-rounded input).
     coeffs: list of (a, b, c) triples, one per step.
+    beside: chain_blocks of the stacks whose chains run at the same time on other streams
+        (the result does not depend on it).
     Returns a contiguous bf16 tensor of the input's shape.
     """
     _require_gpu(X, "ns_chain")
@@ -156,9 +166,10 @@ def ns_chain(X, orient_tall, entry_mode, coeffs, out=None):
     nbytes = ns_workspace_bytes(B, R, C, bool(orient_tall))
     ws = _workspace(nbytes, X.device)
     bs, rs, cs = X.stride()
-    rc = lib.dmh_ns_chain(_stream(X.device), c_vp(X.data_ptr()), 0 if X.dtype == torch.float32 else 1,
-                          B, R, C, bs, rs, cs, c_vp(out.data_ptr()), int(bool(orient_tall)),
-                          int(entry_mode), flat, steps, c_vp(ws.data_ptr()), nbytes)
+    rc = lib.dmh_ns_chain_beside(_stream(X.device), c_vp(X.data_ptr()),
+                                 0 if X.dtype == torch.float32 else 1, B, R, C, bs, rs, cs,
+                                 c_vp(out.data_ptr()), int(bool(orient_tall)), int(entry_mode),
+                                 flat, steps, c_vp(ws.data_ptr()), nbytes, int(beside))
     _check(rc, "dmh_ns_chain")
     return out
 

@@ -61,13 +61,15 @@ def plain_group_chains(stacks, talls, entry_mode, sched):
     # are dropped.  (Shared with record_stream, it would be free once the GPU had got there, and
     # a host that runs ahead would allocate every bucket of a step anew.)
     outs = [torch.empty(X.shape, dtype=torch.bfloat16, device=dev) for X in stacks]
+    blocks = [_native.chain_blocks(X) for X in stacks]
     side = _side_streams(dev, len(stacks))
     for s in side:
         s.wait_stream(main)
     try:
         for s, i in zip(side, order):
             with torch.cuda.stream(s):
-                _native.ns_chain(stacks[i], talls[i], entry_mode, sched, out=outs[i])
+                _native.ns_chain(stacks[i], talls[i], entry_mode, sched, out=outs[i],
+                                 beside=sum(blocks) - blocks[i])
     finally:
         for s in side:
             main.wait_stream(s)

@@ -109,6 +109,20 @@ def test_chain_result_does_not_depend_on_the_batch(N, m):
             assert torch.equal(many[b].view(torch.int16), u[0].view(torch.int16)), (batch, b)
 
 
+@pytest.mark.parametrize("shape", [(1, 64, 64), (2, 65, 33), (3, 100, 300), (1, 1000, 333), (2, 640, 320),
+                                   (5, 448, 448), (2, 1280, 1280)])
+def test_chain_result_does_not_depend_on_what_runs_beside_it(N, shape):
+    """Kernels chosen for a GPU that other chains fill (at the rule's line and far past it) give
+    the bits of the chain alone, whichever of them pads its entry."""
+    X = torch.randn(*shape, generator=torch.Generator(device=DEV).manual_seed(sum(shape)), device=DEV)
+    line = 15000 - N.chain_blocks(X)
+    for tall in (True, False):
+        want = N.ns_chain(X, tall, 2, O.ns_schedule(3))
+        for beside in (1, line - 1, line, 1 << 40):
+            got = N.ns_chain(X, tall, 2, O.ns_schedule(3), beside=beside)
+            assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (tall, beside)
+
+
 def test_zero_steps_and_entry(N):
     G = torch.randn(2, 96, 160, generator=torch.Generator().manual_seed(3))
     for mode, scale in ((1, 1.0), (2, 1.01)):
