@@ -87,7 +87,9 @@ int dmh_ns_chain_noalloc(dmh_stream_t stream, const void* x, int x_dtype, int ba
  * The dtype-preserving path of _horner_iterate (defmuon/optim/deflation_batched.py:
  * 196-204) for fp32 input: per (a, b, c) in coeffs, G = X^T X, B = b G + (c G) G,
  * X <- a X + X B, in fp32 precision (the products as six bf16 MFMA products of
- * three-term splits, summed in fp32).  x, out: (batch, n, m) fp32, contiguous, distinct.
+ * three-term splits, summed in fp32; large batches of small matrices, from 96 of 64 x 32 and
+ * 1024 of 100 x 100 on, by fp32 MFMA, so a matrix's last bits may depend on the size of its
+ * batch).  x, out: (batch, n, m) fp32, contiguous, distinct.
  */
 int dmh_horner_f32_workspace_size(int batch, int n, int m, size_t* bytes);
 int dmh_horner_f32(dmh_stream_t stream, const float* x, int batch, int n, int m, float* out,

@@ -6,7 +6,8 @@
 // hand the iteration fp32 matrices (the reference's own convergence study runs it in
 // fp32), one launch per GEMM phase over the batch.  gemm_split (below) runs it on the bf16
 // matrix cores with split operands; gemm_f32, on the fp32 matrix cores, takes the matrices
-// whose planes gemm_split cannot address.  In gemm_f32 each phase has the reference's
+// whose planes gemm_split cannot address, and large batches of small ones, whose planes would
+// be mostly padding.  In gemm_f32 each phase has the reference's
 // rounding points (c G and b G rounded on their own, each sum of two rounded terms rounded
 // once; gemm_split scales the sum G G by c instead of G):
 //   C[i][j] = fl(fl(beta * R[i][j]) + fl(sum_k fl(s * P(i, k)) Q(j, k)))
@@ -580,13 +581,36 @@ static int launch_split(const SplitGemm& g, int batch, hipStream_t stream, const
   return DMH_OK;
 }
 
-// The split chain addresses a plane with 32-bit offsets; larger matrices, or
-// DMH_HORNER_SPLIT=0 (for comparisons), run on the fp32 matrix cores.
-static bool use_split(int n, int m) {
+// Whether the traffic of planes padded to 128 costs a batch of small matrices more than the
+// split products give: gemm_f32 pads in LDS only.  It is bound by the K walk of a lone tile in
+// a small batch and by its traffic from some hundreds of matrices on, so the line is a batch
+// size.  us for five steps, fp32 cores / split, above the lines: 128 x (32, 32) 112 / 134, 192 x
+// (128, 32) 157 / 173, 256 x (1024, 32) 674 / 694, 384 x (64, 64) 290 / 296, 768 x (200, 64) 715
+// / 801, 1024 x (100, 100) 794 / 881, 2048 x (40, 32) 433 / 1289, (64, 64) 860 / 1385, (100, 100)
+// 1515 / 1682, and (16, 16) in any batch, 1: 76 / 99, 2048: 234 / 1214; below: 64 x (64, 32) 130 /
+// 117, 128 x (1024, 32) 596 / 399, 256 x (64, 64) 222 / 200, 512 x (128, 64) 381 / 366, 768 x (100,
+// 100) 661 / 641, and larger matrices in any batch, 2048 x (256, 100) 2453 / 2404, (130, 130)
+// 7180 / 5973.
+static bool padding_bound(int batch, int n, int m) {
+  const long long nm = (long long)n * m;
+  if (m <= 32) return nm <= 256 || batch >= (n <= 64 ? 96 : n <= 256 ? 192 : 256);
+  if (m <= 64) return batch >= (n <= 64 ? 320 : 576);
+  return n <= S_TILE && m <= S_TILE && 5 * nm <= 4 * S_TILE * S_TILE && batch >= 1024;
+}
+
+// The split chain addresses a plane with 32-bit offsets; larger matrices run on the fp32 matrix
+// cores, as do those it would pad too much.  DMH_HORNER_SPLIT (for comparisons): 0 none, 1 all
+// that it can address.
+static bool use_split(int batch, int n, int m) {
   const char* env = getenv("DMH_HORNER_SPLIT");
   if (env && env[0] == '0') return false;
   const long long np = ceil_div(n, S_TILE) * (long long)S_TILE, mp = ceil_div(m, S_TILE) * (long long)S_TILE;
-  return np * mp * 2 < (1LL << 31) && mp * mp * 2 < (1LL << 31);
+  if (np * mp * 2 >= (1LL << 31) || mp * mp * 2 >= (1LL << 31)) return false;
+  return (env && env[0] == '1') || !padding_bound(batch, n, m);
+}
+
+static size_t gemm_f32_ws(int batch, int n, int m) {
+  return (size_t)batch * (2 * (size_t)m * m + (size_t)n * m) * sizeof(float);
 }
 
 // planes of X (twice), G and B
@@ -638,8 +662,7 @@ static int horner_split(hipStream_t stream, const float* x, int batch, int n, in
 }
 
 static size_t horner_f32_ws(int batch, int n, int m) {
-  if (use_split(n, m)) return split_ws(batch, n, m);
-  return (size_t)batch * (2 * (size_t)m * m + (size_t)n * m) * sizeof(float);
+  return use_split(batch, n, m) ? split_ws(batch, n, m) : gemm_f32_ws(batch, n, m);
 }
 
 }  // namespace dmh
@@ -677,7 +700,8 @@ int dmh_horner_f32(hipStream_t stream, const float* x, int batch, int n, int m, 
     DMH_CHECK_LAUNCH("dmh_horner_f32 copy");
     return DMH_OK;
   }
-  if (use_split(n, m)) return horner_split(stream, x, batch, n, m, out, coeffs, steps, ws);
+  if (use_split(batch, n, m))
+    return horner_split(stream, x, batch, n, m, out, coeffs, steps, ws);
   float* G = (float*)ws;
   float* Bm = G + gsz * batch;
   float* tmp = Bm + gsz * batch;

@@ -244,3 +244,19 @@ def test_horner_fp32_split_is_as_accurate_as_fp32(N, shape, sched, monkeypatch):
         errs[split] = rel(N.horner_f32(X, hs), want)
     assert errs["1"] < 1e-5, errs
     assert errs["1"] <= 1.1 * errs["0"] + 5 * 2.0 ** -24, errs
+
+
+@pytest.mark.parametrize("shape", [(1, 16, 16), (1, 17, 16), (95, 40, 32), (96, 40, 32), (191, 65, 20), (192, 65, 20), (256, 257, 20),
+                                   (319, 64, 64), (320, 64, 64), (575, 65, 33), (576, 65, 33),
+                                   (1023, 16, 128), (1024, 16, 128), (1024, 100, 100), (1024, 129, 65)])
+def test_horner_fp32_batches_of_small_matrices(N, shape):
+    """Both sides of the lines at which padded planes send a batch to the fp32 matrix cores:
+    within the 1e-5 of 64 bits that the fp32 chain is held to."""
+    X = torch.randn(*shape, generator=torch.Generator(device=DEV).manual_seed(sum(shape)), device=DEV)
+    X = X / X.flatten(1).norm(dim=1)[:, None, None]
+    hs = O.ns_schedule(5)
+    want = X.double()
+    for a, b, c in hs:
+        Gm = want.mT.contiguous() @ want
+        want = a * want + want @ (b * Gm + c * (Gm @ Gm))
+    assert rel(N.horner_f32(X, hs), want) < 1e-5
