@@ -23,6 +23,8 @@
 
 #include <stdlib.h>
 
+#include <algorithm>
+
 namespace dmh {
 
 constexpr int F_TILE = 128;
@@ -619,6 +621,16 @@ static size_t split_ws(int batch, int n, int m) {
   return (size_t)batch * 3 * (2 * np * mp + 2 * mp * mp) * sizeof(bf16);
 }
 
+// Matrices taken at a time: the planes are at least 2.25 times what gemm_f32 needs for the same
+// batch, so a batch goes in equal parts whose planes stay within that or within 1 GiB, whichever
+// is more (or one matrix); 1 GiB is ten matrices of (5120, 1280), several rounds of tiles.
+static int split_part(int batch, int n, int m) {
+  const size_t limit = std::max(gemm_f32_ws(batch, n, m), (size_t)1 << 30);
+  const size_t fit = std::min<size_t>(std::max<size_t>(limit / split_ws(1, n, m), 1), 65535);
+  const int parts = (int)((batch + fit - 1) / fit);
+  return parts > 1 ? ceil_div(batch, parts) : batch;
+}
+
 static int horner_split(hipStream_t stream, const float* x, int batch, int n, int m, float* out,
                         const double* coeffs, int steps, void* ws) {
   const int np = ceil_div(n, S_TILE) * S_TILE, mp = ceil_div(m, S_TILE) * S_TILE;
@@ -662,7 +674,7 @@ static int horner_split(hipStream_t stream, const float* x, int batch, int n, in
 }
 
 static size_t horner_f32_ws(int batch, int n, int m) {
-  return use_split(batch, n, m) ? split_ws(batch, n, m) : gemm_f32_ws(batch, n, m);
+  return use_split(batch, n, m) ? split_ws(split_part(batch, n, m), n, m) : gemm_f32_ws(batch, n, m);
 }
 
 }  // namespace dmh
@@ -700,8 +712,15 @@ int dmh_horner_f32(hipStream_t stream, const float* x, int batch, int n, int m, 
     DMH_CHECK_LAUNCH("dmh_horner_f32 copy");
     return DMH_OK;
   }
-  if (use_split(batch, n, m))
-    return horner_split(stream, x, batch, n, m, out, coeffs, steps, ws);
+  if (use_split(batch, n, m)) {
+    const int part = split_part(batch, n, m);
+    for (int b = 0; b < batch; b += part) {
+      const int rc = horner_split(stream, x + b * tsz, std::min(part, batch - b), n, m, out + b * tsz,
+                                  coeffs, steps, ws);
+      if (rc) return rc;
+    }
+    return DMH_OK;
+  }
   float* G = (float*)ws;
   float* Bm = G + gsz * batch;
   float* tmp = Bm + gsz * batch;

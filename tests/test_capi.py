@@ -80,6 +80,21 @@ def test_workspace_sizes_for_empty_batch(lib):
     assert lib.dmh_ns_workspace_size(0, 512, 256, 1, ctypes.byref(n)) == 0
 
 
+@pytest.mark.parametrize("batch,n,m", [(1, 5120, 1280), (8, 1536, 768), (72, 5120, 1280), (144, 1280, 1280),
+                                       (4096, 64, 64), (1000, 40, 32), (95, 17, 16), (100000, 130, 129),
+                                       (1, 1000000, 1), (3, 40000, 8)])
+def test_fp32_iteration_workspace(lib, batch, n, m):
+    """The fp32 iteration needs at most what fp32 G, B and X take, or 1 GiB, or one matrix's
+    bf16 planes padded to 128 (three each of X twice, G and B), whatever the batch."""
+    size = ctypes.c_size_t()
+    assert lib.dmh_horner_f32_workspace_size(batch, n, m, ctypes.byref(size)) == 0
+    np_, mp = -(-n // 128) * 128, -(-m // 128) * 128
+    fp32 = batch * (2 * m * m + n * m) * 4
+    planes = 12 * (np_ * mp + mp * mp)
+    assert size.value <= max(fp32, 1 << 30, planes)
+    assert size.value >= min(fp32, planes)
+
+
 def test_chain_refuses_operands_beyond_32bit_addressing(lib):
     """The bf16 chain addresses each padded operand through 32-bit buffer descriptors
     and offsets: a matrix whose padded bf16 iterate reaches 2^31 bytes is refused with

@@ -260,3 +260,14 @@ def test_horner_fp32_batches_of_small_matrices(N, shape):
         Gm = want.mT.contiguous() @ want
         want = a * want + want @ (b * Gm + c * (Gm @ Gm))
     assert rel(N.horner_f32(X, hs), want) < 1e-5
+
+
+def test_horner_fp32_batch_in_parts(N):
+    """A batch whose planes take more than the workspace goes in parts, the last one shorter:
+    every matrix as by itself, bit for bit."""
+    X = torch.randn(131, 1024, 640, generator=torch.Generator(device=DEV).manual_seed(5), device=DEV)
+    X = X / X.flatten(1).norm(dim=1)[:, None, None]
+    hs = O.pe_schedule(2)
+    got = N.horner_f32(X, hs)
+    for b in range(131):
+        assert torch.equal(got[b], N.horner_f32(X[b:b + 1], hs)[0]), b
