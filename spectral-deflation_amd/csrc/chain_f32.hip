@@ -244,14 +244,15 @@ __host__ __device__ __forceinline__ long long split_off(int i, int j, int R) {
   return ((long long)(j >> 5) * (R >> 6) + (i >> 6)) * 2048 + (i & 63) * 32 + (j & 31);
 }
 
-// x = t[0] + t[1] + t[2]
+// x = t[0] + t[1] + t[2] for |x| >= 2^-102 (below, the last terms run out of exponents); an
+// infinite x gives NaN
 __device__ __forceinline__ void split3(const float (&x)[8], bf16x8 (&t)[3]) {
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     float r = x[e];
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
-      const bf16 h = f2bf(r);
+      const bf16 h = f2bf(p == 0 ? bf16_range(r) : r);
       t[p][e] = h;
       r -= bf2f(h);
     }

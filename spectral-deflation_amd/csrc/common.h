@@ -29,6 +29,13 @@ void set_error(const char* fmt, ...);
 __device__ __forceinline__ bf16 f2bf(float x) { return (bf16)x; }
 __device__ __forceinline__ float bf2f(bf16 x) { return (float)x; }
 
+// x within the finite bf16 range, for the first term of a split: fp32 values from 3.3962e38 on
+// round to infinity, and the next term to NaN.  NaN and infinities give NaN in the later terms.
+__device__ __forceinline__ float bf16_range(float x) {
+  constexpr float M = 3.38953139e38f;
+  return fminf(fmaxf(x, -M), M);
+}
+
 // Map a hardware workgroup id to a logical tile id so that each XCD (the
 // dispatcher deals workgroups round-robin over the 8 XCDs) works on a
 // contiguous range of logical tiles and shares their operands in its L2.

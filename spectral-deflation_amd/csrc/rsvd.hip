@@ -468,14 +468,16 @@ __global__ __launch_bounds__(256) void transpose_rp(const float* __restrict__ sr
 // operand and column l%32 of the second; the result D[8g + 4(l/32) + q][l%32] is
 // acc[4g + q].
 // ---------------------------------------------------------------------------
-template <int SPLITS>
+// The terms' sum is x for 2^-102 <= |x| < 3.3962e38, where bf16 rounds to infinity, or with FULL
+// up to the largest fp32, 3.4028e38 (below 2^-102 the last terms run out of exponents).
+template <int SPLITS, bool FULL = false>
 __device__ __forceinline__ void split_bf16(const float (&x)[8], bf16x8 (&t)[SPLITS]) {
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     float r = x[e];
 #pragma unroll
     for (int s = 0; s < SPLITS; ++s) {
-      const bf16 h = f2bf(r);
+      const bf16 h = f2bf(FULL && s == 0 ? bf16_range(r) : r);
       t[s][e] = h;
       r -= bf2f(h);
     }
@@ -829,7 +831,7 @@ __device__ __forceinline__ void sk_pin(SkStageQ<Q>& st) {
 // order of sk_rows' 16x16 fragments -- within each 32-index step, the 4-index group
 // a = 0..7 at position 8a (a < 4) or 8(a - 4) + 4 (a >= 4), so positions 8g .. 8g + 7
 // hold the indices 4g .. 4g + 3 and 16 + 4g .. 16 + 4g + 3.
-template <int SPLITS, bool PERM = false, int Q = 2>
+template <int SPLITS, bool PERM = false, int Q = 2, bool FULL = false>
 __device__ __forceinline__ void sk_stage_store(const SkStageQ<Q>& st, bf16* buf, int tid) {
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
@@ -838,7 +840,7 @@ __device__ __forceinline__ void sk_stage_store(const SkStageQ<Q>& st, bf16* buf,
     const float x[8] = {st.v[q][0].x, st.v[q][0].y, st.v[q][0].z, st.v[q][0].w,
                         st.v[q][1].x, st.v[q][1].y, st.v[q][1].z, st.v[q][1].w};
     bf16x8 t[SPLITS];
-    split_bf16<SPLITS>(x, t);
+    split_bf16<SPLITS, FULL>(x, t);
     if (PERM) {
       // the 8 indices are the 4-index groups a0 and a0 + 1 (a0 even) of step kk / 32
       const int a0 = (kk & 31) >> 2, step = kk & ~31;
@@ -1279,7 +1281,7 @@ __global__ __launch_bounds__(256) void sk_rows_small(const float* __restrict__ A
   load(0, ab[0]);
   load(1, ab[1]);
   sk_pin(stg);
-  sk_stage_store<SPLITS, true>(stg, xl, tid);
+  sk_stage_store<SPLITS, true, 2, SEP>(stg, xl, tid);
   sk_stage_load(stg, xr, ldxt, SK_KC, m, tid);
   sk_barrier();
   for (int ch = 0; ch < nch; ++ch) {
@@ -1308,13 +1310,13 @@ __global__ __launch_bounds__(256) void sk_rows_small(const float* __restrict__ A
           sq += (double)f;
         }
         bf16x8 as[SPLITS];
-        split_bf16<SPLITS>(v, as);
+        split_bf16<SPLITS, SEP>(v, as);
         if constexpr (SEP) mfma_split16_sep(xs, as, acc[rb], low[rb]);
         else mfma_split16<SPLITS>(xs, as, acc[rb]);
       }
     }
     sk_pin(stg);
-    sk_stage_store<SPLITS, true>(stg, xl + ((ch + 1) & 1) * SK_BUF, tid);
+    sk_stage_store<SPLITS, true, 2, SEP>(stg, xl + ((ch + 1) & 1) * SK_BUF, tid);
     sk_barrier();
     sk_stage_load(stg, xr, ldxt, (ch + 2) * SK_KC, m, tid);
   }
@@ -1339,8 +1341,8 @@ __global__ __launch_bounds__(256) void sk_rows_small(const float* __restrict__ A
 // of A; lane l reads the columns j0 + 2 l32 + {0, 1} of 8 consecutive rows, i.e. two
 // 32-column MFMA blocks (block e holds the columns j0 + 2 l32 + e).  Needs rps % 16 == 0 and
 // YT zero from n to ldyt (a multiple of 8); rows past n load zeros.  ODD (m odd): the lane of
-// the last column alone loads the pair that ends with it.  SEP: mfma_split_sep (the shapes
-// that the fp32 matrix cores had before, whose error it stays below).
+// the last column alone loads the pair that ends with it.  SEP: mfma_split_sep and the whole
+// fp32 range (for what the fp32 matrix cores took before, whose error it stays below).
 template <int SPLITS, bool ODD = false, bool SEP = false>
 __global__ __launch_bounds__(256) void sk_cols(const float* __restrict__ A, int n, int m,
                                                const float* __restrict__ YT, int ldyt, int rps,
@@ -1379,7 +1381,7 @@ __global__ __launch_bounds__(256) void sk_cols(const float* __restrict__ A, int 
   };
   SkStage stg;
   sk_stage_load(stg, yr, ldyt, ib, ie, tid);
-  sk_stage_store<SPLITS>(stg, yl, tid);
+  sk_stage_store<SPLITS, false, 2, SEP>(stg, yl, tid);
   sk_stage_load(stg, yr, ldyt, ib + SK_KC, ie, tid);
   // A two substeps ahead: slot p & 1 holds substep ks (SK_KC / 16 == 4 per chunk)
   static_assert(SK_KC % 32 == 0, "an even number of A substeps per staged chunk");
@@ -1404,8 +1406,8 @@ __global__ __launch_bounds__(256) void sk_cols(const float* __restrict__ A, int 
       {
         const float v0[8] = {ac[0].x, ac[1].x, ac[2].x, ac[3].x, ac[4].x, ac[5].x, ac[6].x, ac[7].x};
         const float v1[8] = {ac[0].y, ac[1].y, ac[2].y, ac[3].y, ac[4].y, ac[5].y, ac[6].y, ac[7].y};
-        split_bf16<SPLITS>(v0, as[0]);
-        split_bf16<SPLITS>(v1, as[1]);
+        split_bf16<SPLITS, SEP>(v0, as[0]);
+        split_bf16<SPLITS, SEP>(v1, as[1]);
       }
       sk_frags<SPLITS>(buf, 16 * p + 8 * hk, l32, ys);
 #pragma unroll
@@ -1418,7 +1420,7 @@ __global__ __launch_bounds__(256) void sk_cols(const float* __restrict__ A, int 
     }
     // (after the last chunk this stages zeros nobody reads: no branch in the loop)
     sk_pin(stg);
-    sk_stage_store<SPLITS>(stg, yl + ((ch + 1) & 1) * SK_BUF, tid);
+    sk_stage_store<SPLITS, false, 2, SEP>(stg, yl + ((ch + 1) & 1) * SK_BUF, tid);
     sk_barrier();
     sk_stage_load(stg, yr, ldyt, ib + (ch + 2) * SK_KC, ie, tid);
   }
@@ -2890,7 +2892,7 @@ static int skr(hipStream_t st, const float* A, int B, int n, int m, const float*
 // C (m x RP) = A^T YT^T with the split-bf16 kernel (YT: RP x sk_pitch(n)), row splits reduced
 // in order
 static int skc(hipStream_t st, const float* A, int B, int n, int m, const float* YT, float* C,
-               const RsvdWs& w) {
+               const RsvdWs& w, bool sep = false) {
   int S, rps;
   sk_splits(B, n, m, &S, &rps);
   dim3 grid(ceil_div(m, SKC_COLS), S, B);
@@ -2898,7 +2900,7 @@ static int skc(hipStream_t st, const float* A, int B, int n, int m, const float*
   if (m % 2)
     hipLaunchKernelGGL((sk_cols<3, true, true>), grid, dim3(256), 0, st, A, n, m, YT, sk_pitch(n),
                        rps, S == 1 ? C : w.part);
-  else if (sk_ragged(n, m))
+  else if (sep || sk_ragged(n, m))
     hipLaunchKernelGGL((sk_cols<3, false, true>), grid, dim3(256), 0, st, A, n, m, YT, sk_pitch(n),
                        rps, S == 1 ? C : w.part);
   else
@@ -3113,7 +3115,11 @@ int dmh_project(hipStream_t stream, const float* Q, const float* A, int batch, i
     hipLaunchKernelGGL(transpose_rp, dim3(ceil_div(n, 64), batch), dim3(256), 0, stream, Q, n, r, r,
                        (long long)n * r, w.QT, sk_pitch(n));
     DMH_CHECK_LAUNCH("transpose Q");
-    rc = skc(stream, A, batch, n, m, w.QT, w.Bt, w);
+    // (SEP for every size: the one product's error is the result's.  Against 64 bits, s and
+    // U S V^T on the fp32 matrix cores / here: (5120, 1280), r = 64, 4.6e-8 and 1.6e-6 / 2.8e-8 and
+    // 9.8e-7; 2 x (1024, 1024), r = 52, 3.2e-8 and 1.05e-6 / 2.6e-8 and 9.0e-7; 4 x (64, 64), r = 8,
+    // 3.5e-8 and 2.9e-7 / 2.9e-8 and 2.6e-7)
+    rc = skc(stream, A, batch, n, m, w.QT, w.Bt, w, true);
   } else {
     rc = sg(stream, SG_COLSTREAM, A, batch, n, m, w.Q, RP, RP, (long long)n * RP, w.Bt,
             (long long)m * RP);

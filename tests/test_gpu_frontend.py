@@ -457,7 +457,28 @@ def test_skinny_products_of_any_width(N, n, m, monkeypatch):
     assert rel(outs[0][5], X0o) < 1e-4
 
 
-@pytest.mark.parametrize("n,m,r", [(40, 13, 13), (1001, 333, 18), (300, 300, 64)])
+@pytest.mark.parametrize("n,m", [(67, 33), (67, 34), (68, 36), (129, 33)])
+@pytest.mark.parametrize("top", [3.3895e38, 3.395e38, 3.4028e38])
+def test_skinny_products_up_to_the_largest_float(N, n, m, top):
+    """Entries that bf16 rounds to infinity (from 3.3962e38 on) keep their value in the split
+    products of sizes that are no multiple of 8, and in dmh_project at any size: equal singular
+    values come out equal and finite (1e-5: fp32)."""
+    A = torch.zeros(2, n, m)
+    A[:, torch.arange(m), torch.arange(m)] = top
+    A[1] = -A[1]
+    r = 8
+    Om = torch.randn(2, m, r, generator=torch.Generator().manual_seed(m)) * 1e-3
+    U, s, V = (t.cpu() for t in N.rsvd(A.to(DEV), Om.to(DEV)))
+    assert torch.allclose(s, torch.full_like(s, top), rtol=1e-5)
+    Q = torch.zeros(2, n, r)
+    Q[:, torch.arange(r), torch.arange(r)] = 1
+    for rows, cols in ((n, m), (n // 8 * 8, 32)):
+        U, s, V = (t.cpu() for t in N.project(Q[:, :rows].contiguous().to(DEV),
+                                              A[:, :rows, :cols].contiguous().to(DEV)))
+        assert torch.allclose(s, torch.full_like(s, top), rtol=1e-5)
+
+
+@pytest.mark.parametrize("n,m,r", [(64, 64, 8), (512, 256, 16), (640, 320, 18), (40, 13, 13), (1001, 333, 18), (300, 300, 64)])
 def test_project_of_any_width(N, n, m, r):
     """Rayleigh-Ritz on the split products: s and the reconstruction Q Q^T A = U S V^T against
     fp64 (1e-5: fp32 sums over n, and U and V in fp32)."""
