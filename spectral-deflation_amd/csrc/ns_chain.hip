@@ -125,7 +125,7 @@ struct GemmArgs {
   int total_tiles;                               // over the batch
   int batch, rev;                                // rev: walk the batch from its last matrix
   int kspread;                                   // K walk starts at stage kspread (ti + tj) mod nk
-  int kvalid, ref_tile;                          // gemm_tile64: K without its zero padding, and the
+  int kvalid, ref_tile;                          // gemm_ring: K without its zero padding, and the
                                                  // tile size whose K walk it follows
   float alpha, beta;                             // POLY: (b, c)
   float diag_add; int diag_lim;                  // POLY: + diag_add on C[i][i], i < diag_lim
@@ -745,12 +745,8 @@ __device__ __forceinline__ void wait_vmcnt() {
 // ... for n = k * STEP, k < NS
 template <int STEP, int NS>
 __device__ __forceinline__ void wait_stages(int k) {
-  static_assert(NS <= 8, "cases");
+  static_assert(NS <= 4, "cases");
   switch (k) {
-    case 7: if constexpr (NS > 7) { wait_vmcnt<7 * STEP>(); break; }
-    case 6: if constexpr (NS > 6) { wait_vmcnt<6 * STEP>(); break; }
-    case 5: if constexpr (NS > 5) { wait_vmcnt<5 * STEP>(); break; }
-    case 4: if constexpr (NS > 4) { wait_vmcnt<4 * STEP>(); break; }
     case 3: if constexpr (NS > 3) { wait_vmcnt<3 * STEP>(); break; }
     case 2: if constexpr (NS > 2) { wait_vmcnt<2 * STEP>(); break; }
     case 1: wait_vmcnt<STEP>(); break;
@@ -1392,7 +1388,10 @@ static void chain_cfg(const ChainDims& d, int batch, long long beside, int cfg[3
     for (int i = 0; i < 3; ++i) cfg[i] = c[i] >= RING_NONE && c[i] <= RING_128 ? c[i] : RING_NONE;
 }
 
-// with every phase on gemm_ring nothing past the last 64 x 64 block is read
+// With every phase on gemm_ring nothing past the last 64 x 64 block enters a result.  The
+// 128-wide tiles do read the block after it where the count is odd (inside the padding to 256,
+// so inside the workspace, as it was left), as rows, columns or added terms of outputs past that
+// block, which stay there; K walks stop before it.
 static bool all_ring(const int cfg[3]) { return cfg[0] && cfg[1] && cfg[2]; }
 
 void chain_extent(const ChainDims& d, int batch, int* rows, int* cols, long long beside) {
@@ -1563,7 +1562,7 @@ int dmh_ns_chain(hipStream_t stream, const void* x, int x_dtype, int batch, int 
 // device address: its address on the current device comes from hipGetSymbolAddress,
 // once per device, and only that pointer is handed to kernels.  Every call on a GPU
 // uses the same array, so calls that overlap on one GPU (other streams, other
-// threads) race; the chain writes every byte of its workspace it reads, so nothing
+// threads) race; the chain writes all of its workspace that a result depends on, so nothing
 // needs clearing between calls.
 // ---------------------------------------------------------------------------
 namespace dmh {

@@ -478,6 +478,23 @@ def test_skinny_products_up_to_the_largest_float(N, n, m, top):
         assert torch.allclose(s, torch.full_like(s, top), rtol=1e-5)
 
 
+@pytest.mark.parametrize("n,m", [(128, 64), (100, 100), (257, 66), (131, 131)])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+def test_non_finite_entry_is_declined(N, n, m, bad):
+    """A matrix with an entry that is not finite is declined (k = 0), beside one that is whole
+    and comes out as it does alone."""
+    from defmuon_amd import synthetic as S
+    A = torch.stack([S.spiked_matrix(n, m, seed=b, n_spikes=1, hi=50.0, lo=20.0) for b in range(2)])
+    r, kw = O.sketch_dims(m)
+    Om = O.draw_omega(2, m, r, 3)
+    args = (kw, O.GATE_RATIO, O.DEFLATE_THRESH, O.DIVISOR_PAD)
+    whole = N.rmfro_clip(A[1:].to(DEV), Om[1:].to(DEV), *args)
+    A[0, n - 1, m - 1] = bad
+    X0, k, d = N.rmfro_clip(A.to(DEV), Om.to(DEV), *args)
+    assert k[0].item() == 0
+    assert k[1].item() == whole[1].item() and torch.equal(X0[1:], whole[0]) and torch.equal(d[1:], whole[2])
+
+
 @pytest.mark.parametrize("n,m,r", [(64, 64, 8), (512, 256, 16), (640, 320, 18), (40, 13, 13), (1001, 333, 18), (300, 300, 64)])
 def test_project_of_any_width(N, n, m, r):
     """Rayleigh-Ritz on the split products: s and the reconstruction Q Q^T A = U S V^T against

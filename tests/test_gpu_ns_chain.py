@@ -123,6 +123,38 @@ def test_chain_result_does_not_depend_on_what_runs_beside_it(N, shape):
             assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (tall, beside)
 
 
+@pytest.mark.parametrize("ring", [None, "1_1_2", "3_3_3", "4_4_4", "3_1_2"])
+@pytest.mark.parametrize("shape", [(1, 64, 64), (2, 192, 192), (3, 65, 33), (1, 321, 320), (2, 100, 300), (1, 1088, 577)])
+def test_workspace_contents_stay_out_of_the_result(N, shape, ring, monkeypatch):
+    """A workspace full of NaN, at sizes that leave the 128-wide tiles a block past the matrix
+    (an odd count of 64-blocks): the chain and the deflated front-end and chain give the
+    persistent kernel's bits, entry norm and zero padding included."""
+    g = torch.Generator(device=DEV).manual_seed(sum(shape))
+    X = torch.randn(*shape, generator=g, device=DEV)
+    A = X if shape[1] >= shape[2] else X.mT.contiguous()
+    r, kw = O.sketch_dims(A.shape[2])
+    A = A + 40 * torch.ones_like(A[:1])          # one direction above the gate
+    Om = torch.randn(A.shape[0], A.shape[2], r, generator=g, device=DEV)
+
+    def run():
+        outs = [N.ns_chain(X, tall, 1, O.ns_schedule(3)) for tall in (True, False)]
+        front = N.deflated_polar_front(A, Om, kw, O.GATE_RATIO, O.DEFLATE_THRESH, O.DIVISOR_PAD)
+        outs.append(N.deflated_polar_chain(front, O.ns_schedule(3)))
+        return [t.view(torch.int16) for t in outs] + [front.k, front.d]
+
+    monkeypatch.setenv("DMH_CHAIN_RING", "0_0_0")
+    want = run()
+    assert all(torch.isfinite(t.view(torch.bfloat16).float()).all() for t in want[:3])
+    if ring is None:
+        monkeypatch.delenv("DMH_CHAIN_RING")
+    else:
+        monkeypatch.setenv("DMH_CHAIN_RING", ring)
+    monkeypatch.setattr(N, "_workspace", lambda nbytes, device: torch.full(
+        (max(int(nbytes), 1),), 255, dtype=torch.uint8, device=device))
+    for got, ref in zip(run(), want):
+        assert torch.equal(got, ref)
+
+
 def test_zero_steps_and_entry(N):
     G = torch.randn(2, 96, 160, generator=torch.Generator().manual_seed(3))
     for mode, scale in ((1, 1.0), (2, 1.01)):
