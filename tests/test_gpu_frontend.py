@@ -380,6 +380,28 @@ def test_skinny_rows_direct_to_lds_matches_register_kernel(N, B, n, m, monkeypat
     assert rel(X0, X0r) < 1e-6
 
 
+@pytest.mark.parametrize("B,n,m", [(1, 64, 64), (2, 200, 72), (3, 264, 200), (2, 512, 256), (1, 1000, 320)])
+def test_skinny_rows_small_matches_the_256_row_kernels(N, B, n, m, monkeypatch):
+    """16, 32 and 64 rows per workgroup against 256 (direct-to-LDS where m % 64 == 0, the
+    register kernel elsewhere), at sizes that leave row blocks and 64-index chunks short: U, s,
+    V and k bit for bit, the divisor (its sums of squares in another order) and X0 to fp32
+    rounding."""
+    from defmuon_amd import synthetic as S
+    A = torch.stack([S.spiked_matrix(n, m, seed=9 * b + n, n_spikes=2 if m > 64 else 1, hi=40.0, lo=20.0)
+                     for b in range(B)]).to(DEV)
+    r, kw = O.sketch_dims(m)
+    Om = O.draw_omega(B, m, r, 23).to(DEV)
+    outs = {}
+    for rows in ("256", "16", "32", "64"):
+        monkeypatch.setenv("DMH_SKR_ROWS", rows)
+        X0, k, d = N.rmfro_clip(A, Om, kw, O.GATE_RATIO, O.DEFLATE_THRESH, O.DIVISOR_PAD)
+        outs[rows] = (*N.rsvd(A, Om), k, d, X0)
+    for rows in ("16", "32", "64"):
+        for x, y in zip(outs[rows][:4], outs["256"][:4]):
+            assert torch.equal(x, y), rows
+        assert rel(outs[rows][4], outs["256"][4]) < 1e-6 and rel(outs[rows][5], outs["256"][5]) < 1e-6
+
+
 @pytest.mark.parametrize("kind", ["spiked", "orthonormal", "axes"])
 @pytest.mark.parametrize("m", [1, 2, 3, 40, 41, 160, 161, 321, 1280])
 def test_clip_sketch_width_edges(N, m, kind):

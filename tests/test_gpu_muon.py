@@ -219,33 +219,92 @@ def test_polar_groups_equal_per_group_calls(arm):
 
 
 @pytest.mark.parametrize("arm", ["ns5", "polarexpress"])
-def test_grouped_plain_step_equals_per_parameter_loop(muon_mod, arm):
-    """grouped_plain.install(): one launch per (shape, dtype, orientation) group
-    moves every parameter bit for bit like the per-parameter loop
-    (muon.py:361-386), over two steps (momentum buffers included)."""
+def test_grouped_plain_step_equals_per_parameter_loop(muon_mod, monkeypatch, arm):
+    """grouped_plain.install(): one launch per (shape, dtype, orientation) group of the whole
+    model, where the buckets' limit would have given every parameter its own, moves every
+    parameter bit for bit like the per-parameter loop (muon.py:361-386; a wrapped factorizer
+    keeps it), over two steps (momentum buffers included)."""
     muon, DB = muon_mod
+    from defmuon_amd import _native
     from defmuon_amd.optim import grouped_plain
-    results = {}
-    for grouped in (False, True):
-        if grouped:
+    calls = []
+    chain = _native.ns_chain
+    monkeypatch.setattr(_native, "ns_chain", lambda *a, **kw: calls.append(1) or chain(*a, **kw))
+    results, launches = {}, {}
+    for how in ("loop", "buckets", "grouped"):
+        if how == "grouped":
             grouped_plain.install()
-        else:
-            grouped_plain.uninstall()
         try:
             params = _named_params(7)
             grads = _grads(params, 8)
             opt = muon.Muon(list(params.items()), lr=0.01, weight_decay=0.1, momentum=0.95,
                             nesterov=True, ns_steps=5, polar_method=arm)
+            opt.PLAIN_BUCKET = 0
+            if how == "loop":
+                fac = opt.polar_factorizer
+                opt.polar_factorizer = lambda G, steps: fac(G, steps)
+            calls.clear()
             for _ in range(2):
                 for k, p in params.items():
                     p.grad = grads[k]
                 opt.step()
             torch.cuda.synchronize()
-            results[grouped] = {k: v.detach().clone() for k, v in params.items()}
+            launches[how] = len(calls)
+            results[how] = [p.detach() for p in params.values()] + [
+                opt.state[p]["momentum_buffer"] for p in params.values()
+                if "momentum_buffer" in opt.state[p]]
         finally:
             grouped_plain.uninstall()
-    for k in results[False]:
-        assert torch.equal(results[False][k], results[True][k]), k
+    # three groups: D x D (c_attn's blocks and c_proj), 4D x D and D x 4D
+    assert launches == {"loop": 2 * 4 * LAYERS, "buckets": 2 * 4 * LAYERS, "grouped": 2 * 3}
+    for how in ("buckets", "grouped"):
+        for x, y in zip(results["loop"], results[how]):
+            assert torch.equal(x, y), how
+
+
+@pytest.mark.parametrize("arm", ["ns5", "polarexpress"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_plain_step_under_capture(muon_mod, arm, dtype):
+    """The plain step, several groups of it, captured into a graph on one stream (no side
+    stream joins the capture): every replay, with new gradients in place and eager steps of a
+    twin in between, leaves parameters and momenta bit for bit where the eager step does."""
+    muon, DB = muon_mod
+
+    def model():
+        g = torch.Generator().manual_seed(41)
+        shapes = [(3 * D, D), (D, D), (4 * D, D), (D, 4 * D), (77, 131)]
+        ps = [torch.nn.Parameter(torch.randn(*s, generator=g).to(DEV, dtype)) for s in shapes]
+        for p in ps:
+            p.grad = torch.zeros_like(p)
+        names = ["h.attn.c_attn.weight", "a.weight", "b.weight", "c.weight", "d.weight"]
+        return ps, muon.Muon(list(zip(names, ps)), lr=0.01, weight_decay=0.1, polar_method=arm)
+
+    def new_grads(params, seed):
+        g = torch.Generator().manual_seed(seed)
+        for p in params:
+            p.grad.copy_(torch.randn(p.shape, generator=g).to(DEV, dtype))
+
+    ps, opt = model()
+    qs, twin = model()
+    for params, o in ((ps, opt), (qs, twin)):
+        new_grads(params, 0)
+        o.step()
+    before = [p.detach().clone() for p in ps]
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        opt.step()
+    torch.cuda.synchronize()
+    assert all(torch.equal(p.detach(), b) for p, b in zip(ps, before))   # captured, not run
+    for replay in range(1, 5):
+        new_grads(ps, replay)
+        new_grads(qs, replay)
+        graph.replay()
+        twin.step()
+        torch.cuda.synchronize()
+        for p, q in zip(ps, qs):
+            assert torch.equal(p.detach(), q.detach()), replay
+            assert torch.equal(opt.state[p]["momentum_buffer"], twin.state[q]["momentum_buffer"])
 
 
 @pytest.mark.parametrize("arm", ["ns5", "polarexpress"])
