@@ -76,14 +76,6 @@ def plain_group_chains(stacks, talls, entry_mode, sched):
     return outs
 
 
-def _byte_range(p):
-    """[first, end) of the memory p's elements lie in."""
-    lo = p.data_ptr()
-    if p.numel() == 0:
-        return lo, lo
-    return lo, lo + (1 + sum((n - 1) * st for n, st in zip(p.shape, p.stride()))) * p.element_size()
-
-
 _EXCLUDED = ("embeddings", "embed_tokens", "wte", "lm_head", "wpe")
 
 
@@ -183,15 +175,12 @@ class Muon(torch.optim.Optimizer):
             if plan is not None:
                 mode, sched = plan
                 for bucket in self._plain_buckets(params, mode):
-                    stacks = {}
-                    for p in bucket:
-                        X, tall = self._plain_view(p, p, mode)
-                        key = (tuple(X.shape[1:]), X.dtype, tall)
-                        stacks[key] = stacks.get(key, 0) + X.shape[0]
+                    groups = self._plain_groups(bucket)
                     plain_group_chains(
-                        [torch.zeros((nb,) + shape, dtype=dtype, device=bucket[0].device)
-                         for (shape, dtype, _), nb in stacks.items()],
-                        [tall for _, _, tall in stacks], mode, sched)
+                        [torch.zeros((sum(e["nb"] for e in es),) + shape, dtype=dtype,
+                                     device=es[0]["p"].device)
+                         for (shape, dtype, _), es in groups.items()],
+                        [tall for _, _, tall in groups], mode, sched)
             for p in params:
                 shape = tuple(self._qkv_split(p, p).shape)
                 key = (shape, p.dtype, p.device)
@@ -238,11 +227,14 @@ class Muon(torch.optim.Optimizer):
             g = p.grad
             if g is None:
                 continue
-            buf = self.state[p].get("momentum_buffer")
-            ts = (p.data, g) if buf is None else (p.data, g, buf)
-            if any(not t.is_cuda or t.dtype != torch.float32 or not t.is_contiguous()
-                   or t.shape != p.shape or t.device != p.device for t in ts) or p.ndim != 2:
+            shape, device = p.shape, p.device
+            if len(shape) != 2 or not p.is_cuda:
                 return False
+            buf = self.state[p].get("momentum_buffer")
+            for t in (p, g) if buf is None else (p, g, buf):
+                if (t.dtype != torch.float32 or not t.is_contiguous() or t.shape != shape
+                        or t.device != device):
+                    return False
         return True
 
     def _muon_step_batched(self, group, params, lr, weight_decay, momentum):
@@ -365,7 +357,7 @@ class Muon(torch.optim.Optimizer):
     GROUPED_PLAIN = False   # grouped_plain.install(): buckets of any size
 
     # Bytes that the parameters sharing a plain-arm step's launches take beside their gradients
-    # and state (_plain_bytes).  A chain alone on one GPT-2-small matrix leaves most compute
+    # and state (_plain_entry).  A chain alone on one GPT-2-small matrix leaves most compute
     # units idle (about 170 us each, sixteen in a row for four layers: a step 2980 us one by one,
     # 1036 in a bucket; one layer of width 64 is bound by its launches, 754 at one factorizer
     # call each, 540 here).  1 GiB is nine GPT-2-small layers or three of GPT-2 large, several
@@ -381,50 +373,58 @@ class Muon(torch.optim.Optimizer):
             return 2, pe_schedule(steps)
         return None
 
-    def _plain_view(self, p, t, mode):
-        """The matrices the factorizer takes t (p's momentum, or p itself) for, as a batch, and
-        their orientation (size(0) > size(1) for ns5, muon.py:30; size(-2) > size(-1) for
-        PolarExpress, polar_express.py:25)."""
-        q = self._qkv_split(p, t)
-        tall = q.size(0) > q.size(1) if mode == 1 else q.size(-2) > q.size(-1)
-        return as_batch(q), tall
-
-    def _plain_bytes(self, p, mode):
-        """At most what p adds to its bucket: momentum, stack and polar factor, and the chain's
-        workspace, which pads the matrices (a 4096 x 8 one takes 4.3 MB)."""
-        if p.numel() == 0:
-            return 0
-        X, tall = self._plain_view(p, p, mode)
-        return (p.numel() * (2 * max(p.element_size(), 4) + 2)
-                + _native.ns_workspace_bytes(*X.shape, tall))
+    def _plain_entry(self, p, mode):
+        """What a plain step has to know of a parameter: the matrices its factorizer takes, their
+        orientation (size(0) > size(1) for ns5, muon.py:30; size(-2) > size(-1) for
+        PolarExpress, polar_express.py:25), and the bytes that it adds to its bucket at most:
+        momentum, stack and polar factor, and the chain's workspace, which pads the matrices (a
+        4096 x 8 one takes 4.3 MB)."""
+        s = self._qkv_split(p, p if p.grad is None else p.grad).shape
+        tall = s[0] > s[1] if mode == 1 else s[-2] > s[-1]
+        nb, shape = (1 if len(s) == 2 else math.prod(s[:-2])), (s[-2], s[-1])
+        need = p.numel() * (18 if p.dtype is torch.float64 else 10)
+        if need:
+            need += _native.ns_workspace_bytes(nb, s[-2], s[-1], tall)
+        return {"p": p, "tr": False, "nb": nb, "key": (shape, p.dtype, tall)}, need
 
     def _plain_buckets(self, params, mode):
-        """`params` in runs of at most PLAIN_BUCKET bytes on one
-        device, in their order.  Parameters that share memory (one given twice, tied
-        weights) come in buckets of their own: a bucket reads and writes all of its
-        parameters at once, where the loop takes one after the other."""
-        buckets, size = [], 0
+        """The entries of `params` in runs of at most PLAIN_BUCKET bytes on one device, in
+        their order.  Parameters that share memory (one given twice, tied weights) come in
+        buckets of their own: a bucket reads and writes all of its parameters at once, where
+        the loop takes one after the other."""
+        buckets, device = [], None
+        limit = math.inf if self.GROUPED_PLAIN else self.PLAIN_BUCKET
         for p in params:
-            lo, hi = _byte_range(p)
-            need = self._plain_bytes(p, mode)
+            e, need = self._plain_entry(p, mode)
+            lo, span = p.data_ptr(), p.numel()    # p's elements lie in [lo, hi)
+            if span and not p.is_contiguous():
+                span = 1 + sum((n - 1) * st for n, st in zip(p.shape, p.stride()))
+            hi = lo + span * p.element_size()
             if buckets:
                 i = bisect.bisect(los, lo)
                 shares = (i > 0 and his[i - 1] > lo) or (i < len(los) and los[i] < hi)
-            if (not buckets or p.device != buckets[-1][0].device or shares
-                    or (size + need > self.PLAIN_BUCKET and not self.GROUPED_PLAIN)):
+            if not buckets or shares or size + need > limit or p.device != device:
                 buckets.append([])
-                size, los, his, i = 0, [], [], 0
-            buckets[-1].append(p)
+                device, size, los, his, i = p.device, 0, [], [], 0
+            buckets[-1].append(e)
             size += need
             los.insert(i, lo)     # the ranges of a bucket, disjoint and in order
             his.insert(i, hi)
         return buckets
 
+    @staticmethod
+    def _plain_groups(bucket):
+        """A bucket's entries by (matrix shape, dtype, orientation)."""
+        groups = {}
+        for e in bucket:
+            groups.setdefault(e["key"], []).append(e)
+        return groups
+
     def _muon_step_plain_grouped(self, group, params, lr, weight_decay, momentum):
         """The plain-arm update (muon.py:361-386) with one library launch per
         (matrix shape, dtype, orientation) of a bucket of parameters instead of one
         factorizer call per parameter.  The orientation is the one the factorizer itself
-        would pick for the parameter (_plain_view), the entry normalisation is per matrix,
+        would pick for the parameter (_plain_entry), the entry normalisation is per matrix,
         and the matrices of a launch do not interact, so every update equals the
         per-parameter one.  Returns False (nothing done) for a factorizer other than the
         built-in two."""
@@ -437,26 +437,28 @@ class Muon(torch.optim.Optimizer):
             self._plain_bucket_step(group, bucket, lr, weight_decay, momentum, mode, sched)
         return True
 
-    def _plain_bucket_step(self, group, params, lr, weight_decay, momentum, mode, sched):
-        fused = self._fused_glue_ok(group, params)
-        groups = {}
-        for p in params:
-            g = p.grad
+    def _plain_bucket_step(self, group, bucket, lr, weight_decay, momentum, mode, sched):
+        fused = self._fused_glue_ok(group, [e["p"] for e in bucket])
+        if not fused:
+            bucket = [dict(e) for e in bucket]   # (theirs end with the call, and their tensors)
+        for e in bucket:
+            p, g = e["p"], e["p"].grad
             state = self.state[p]
             if "momentum_buffer" not in state:
                 state["momentum_buffer"] = torch.zeros_like(g)
             if not fused:
                 buf = state["momentum_buffer"]
                 buf.mul_(momentum).add_(g)
-                g = g.add(buf, alpha=momentum) if group["nesterov"] else buf
-            X, tall = self._plain_view(p, g, mode)
-            e = {"p": p, "g": g, "X": X, "tr": False, "nb": X.shape[0]}
-            groups.setdefault((tuple(X.shape[1:]), X.dtype, tall), []).append(e)
+                e["g"] = g.add(buf, alpha=momentum) if group["nesterov"] else buf
+                e["X"] = as_batch(self._qkv_split(p, e["g"]))
+                shape, _, tall = e["key"]     # (a momentum of its own dtype decides)
+                e["key"] = shape, e["X"].dtype, tall
+        groups = self._plain_groups(bucket)
         stacks = []
         for (shape, _, _), es in groups.items():
-            if fused:   # momentum and stack in one launch; X is not read
+            if fused:   # momentum and stack in one launch
                 X = torch.empty((sum(e["nb"] for e in es),) + shape, dtype=torch.float32,
-                                device=params[0].device)
+                                device=es[0]["p"].device)
                 _native.momentum_stack(self._glue_params(es, shape), momentum,
                                        group["nesterov"], X)
             else:

@@ -313,7 +313,8 @@ def test_plain_step_under_capture(muon_mod, arm, dtype):
 def test_plain_buckets_equal_factorizer_calls(muon_mod, arm, dtype, bucket):
     """Buckets of any size move every parameter and momentum bit for bit like one
     factorizer call per parameter (a wrapped factorizer keeps that loop), W_QKV, ragged and
-    strided parameters among them; a parameter without a gradient stays."""
+    strided parameters and one with an fp32 momentum among them; a parameter without a gradient
+    stays."""
     muon, DB = muon_mod
     results = {}
     for loop in (True, False):
@@ -332,6 +333,8 @@ def test_plain_buckets_equal_factorizer_calls(muon_mod, arm, dtype, bucket):
             opt.polar_factorizer = lambda G, steps: fac(G, steps)
         elif bucket is not None:
             opt.PLAIN_BUCKET = bucket
+        own = params["h.1.mlp.c_fc.weight"]
+        opt.state[own]["momentum_buffer"] = torch.zeros(own.shape, device=DEV)
         for _ in range(2):
             for k, p in params.items():
                 if k != "idle.weight":

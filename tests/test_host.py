@@ -113,7 +113,7 @@ class _Fake:
         self.shape, self.ndim, self.dtype = torch.Size(shape), len(shape), dtype
         self.device, self.is_cuda = torch.device(device), device.startswith("cuda")
         self.is_contiguous = lambda: contiguous
-        self.data, self.grad = self, None
+        self.grad = None
 
 
 @pytest.mark.parametrize("which", ["grad", "momentum_buffer"])
@@ -154,7 +154,7 @@ def test_plain_buckets_keep_shared_memory_apart():
     def buckets(*params):
         for p in params:
             p.grad = torch.zeros_like(p)
-        return [[id(p) for p in b] for b in opt._plain_buckets(params, 1)]
+        return [[id(e["p"]) for e in b] for b in opt._plain_buckets(params, 1)]
 
     def ids(*groups):
         return [[id(p) for p in g] for g in groups]
@@ -192,7 +192,7 @@ def test_plain_buckets_count_padded_bytes(shape, mode):
     for limit in (0, allocated(1), allocated(3) + 100000, allocated(10) + 100000):
         opt.PLAIN_BUCKET = limit
         bs = opt._plain_buckets(params, mode)
-        assert [id(p) for b in bs for p in b] == [id(p) for p in params]
+        assert [id(e["p"]) for b in bs for e in b] == [id(p) for p in params]
         for b in bs:
             assert len(b) == 1 or allocated(len(b)) <= limit
         assert all(allocated(len(b) + 1) > limit - 10 * 4096 for b in bs[:-1])
