@@ -8,9 +8,11 @@ plain torch tensors); kernels are enqueued on torch's current HIP stream and
 nothing here synchronises.
 """
 
+import contextlib
 import ctypes
 import functools
 import os
+import threading
 
 import torch
 
@@ -133,11 +135,26 @@ def ns_workspace_bytes(batch, rows, cols, orient_tall):
 
 
 def chain_blocks(X):
-    """64 x 64 blocks of a (batch, rows, cols) stack: what ns_chain's `beside` counts."""
+    """64 x 64 blocks of a (batch, rows, cols) stack: what running_beside counts."""
     return X.shape[0] * -(-X.shape[1] // 64) * -(-X.shape[2] // 64)
 
 
-def ns_chain(X, orient_tall, entry_mode, coeffs, out=None, beside=0):
+_beside = threading.local()
+
+
+@contextlib.contextmanager
+def running_beside(blocks):
+    """The calling thread's ns_chain calls inside run at the same time as chains over `blocks`
+    64 x 64 blocks on other streams.  It decides their kernels, never their results."""
+    before = getattr(_beside, "blocks", 0)
+    _beside.blocks = blocks
+    try:
+        yield
+    finally:
+        _beside.blocks = before
+
+
+def ns_chain(X, orient_tall, entry_mode, coeffs, out=None):
     """Run the bf16 polynomial chain on a (batch, rows, cols) stack.
 
     orient_tall: the input is the tall operand T of the tall convention
@@ -146,8 +163,6 @@ def ns_chain(X, orient_tall, entry_mode, coeffs, out=None, beside=0):
     entry_mode: 0 none (input already normalised), 1 divide by ||X||_F + 1e-7,
         2 divide by 1.01 ||X||_F + 1e-7 (norm over the un-rounded input).
     coeffs: list of (a, b, c) triples, one per step.
-    beside: chain_blocks of the stacks whose chains run at the same time on other streams
-        (the result does not depend on it).
     Returns a contiguous bf16 tensor of the input's shape.
     """
     _require_gpu(X, "ns_chain")
@@ -169,7 +184,8 @@ def ns_chain(X, orient_tall, entry_mode, coeffs, out=None, beside=0):
     rc = lib.dmh_ns_chain_beside(_stream(X.device), c_vp(X.data_ptr()),
                                  0 if X.dtype == torch.float32 else 1, B, R, C, bs, rs, cs,
                                  c_vp(out.data_ptr()), int(bool(orient_tall)), int(entry_mode),
-                                 flat, steps, c_vp(ws.data_ptr()), nbytes, int(beside))
+                                 flat, steps, c_vp(ws.data_ptr()), nbytes,
+                                 getattr(_beside, "blocks", 0))
     _check(rc, "dmh_ns_chain")
     return out
 

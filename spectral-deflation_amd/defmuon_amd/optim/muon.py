@@ -67,9 +67,8 @@ def plain_group_chains(stacks, talls, entry_mode, sched):
         s.wait_stream(main)
     try:
         for s, i in zip(side, order):
-            with torch.cuda.stream(s):
-                _native.ns_chain(stacks[i], talls[i], entry_mode, sched, out=outs[i],
-                                 beside=sum(blocks) - blocks[i])
+            with torch.cuda.stream(s), _native.running_beside(sum(blocks) - blocks[i]):
+                _native.ns_chain(stacks[i], talls[i], entry_mode, sched, out=outs[i])
     finally:
         for s in side:
             main.wait_stream(s)

@@ -119,7 +119,8 @@ def test_chain_result_does_not_depend_on_what_runs_beside_it(N, shape):
     for tall in (True, False):
         want = N.ns_chain(X, tall, 2, O.ns_schedule(3))
         for beside in (1, line - 1, line, 1 << 40):
-            got = N.ns_chain(X, tall, 2, O.ns_schedule(3), beside=beside)
+            with N.running_beside(beside):
+                got = N.ns_chain(X, tall, 2, O.ns_schedule(3))
             assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (tall, beside)
 
 
