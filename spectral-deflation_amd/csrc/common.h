@@ -33,7 +33,7 @@ __device__ __forceinline__ float bf2f(bf16 x) { return (float)x; }
 // round to infinity, and the next term to NaN.  NaN and infinities give NaN in the later terms.
 __device__ __forceinline__ float bf16_range(float x) {
   constexpr float M = 3.38953139e38f;
-  return fminf(fmaxf(x, -M), M);
+  return __builtin_amdgcn_fmed3f(x, -M, M);
 }
 
 // Map a hardware workgroup id to a logical tile id so that each XCD (the
