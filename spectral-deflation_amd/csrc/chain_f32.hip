@@ -244,15 +244,16 @@ __host__ __device__ __forceinline__ long long split_off(int i, int j, int R) {
   return ((long long)(j >> 5) * (R >> 6) + (i >> 6)) * 2048 + (i & 63) * 32 + (j & 31);
 }
 
-// x = t[0] + t[1] + t[2] for |x| >= 2^-102 (below, the last terms run out of exponents); an
-// infinite x gives NaN
+// x = t[0] + t[1] + t[2] for 2^-102 <= |x| < 3.3962e38 (below, the last terms run out of
+// exponents).  Larger and infinite x give NaN: the square of one is infinite in G, so no result
+// is finite on the fp32 matrix cores either.
 __device__ __forceinline__ void split3(const float (&x)[8], bf16x8 (&t)[3]) {
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     float r = x[e];
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
-      const bf16 h = f2bf(p == 0 ? bf16_range(r) : r);
+      const bf16 h = f2bf(r);
       t[p][e] = h;
       r -= bf2f(h);
     }
